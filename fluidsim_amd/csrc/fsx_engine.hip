@@ -32,7 +32,7 @@ int fsx_plan_create(fsx_plan* out, int dim, int nx, int ny, int nz, double Lx,
     return fail(FSX_ERR_ARG, "grid dimensions must be >= 2");
   // power-of-two axes: register/LDS Stockham passes; other lengths:
   // mixed-radix passes with two LDS tile buffers (half the length)
-  const int tile = (precision == 4 ? kEPT32 : kEPT64) * kThr;
+  const int tile = precision == 4 ? strided_tile<float>() : strided_tile<double>();
   auto axis_max = [&](int n) { return is_pow2(n) ? tile : tile / 2; };
   if (ny > axis_max(ny) || nz > axis_max(nz) || (is_pow2(nx) ? nx / 2 > tile : nx > tile / 2))
     return fail(FSX_ERR_ARG, "grid dimension too large for the LDS tile");
@@ -87,6 +87,10 @@ int fsx_plan_create(fsx_plan* out, int dim, int nx, int ny, int nz, double Lx,
         if (any[i]) lo = i + 1;
       for (int i = n - 1; i > n / 2; --i)
         if (any[i]) hi = n - i;
+      // a kept Nyquist index without all of the negative ones: keep the
+      // whole axis (the mask prunes), so that a pruned axis of even length
+      // keeps only indices below n / 2 in its lower range (fsx_tile.h)
+      if (n % 2 == 0 && lo == n / 2 + 1) hi = n - lo;
       return AxisMap{n, lo, hi};
     };
     if (nkept == 0) mx = 1;

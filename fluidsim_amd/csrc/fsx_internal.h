@@ -185,17 +185,9 @@ int tm_flush(fsx_plan_s* p) {
   return 0;
 }
 
-constexpr int kThr = 512;   // threads per workgroup of the strided passes
 constexpr int kXThr = 512;       // threads per workgroup of the LDS row pass
-constexpr int kXPassEptDiv = 2;  // its tile: half the strided passes' elements per thread
-constexpr int kEPT32 = 16;  // 8192 complex64 per tile  = 64 KiB of LDS
-constexpr int kEPT64 = 8;   // 4096 complex128 per tile = 64 KiB of LDS
+constexpr int kXPassE = 8;       // elements per thread of its tile
 constexpr int kMinBlocks = 1024;  // shrink tiles of small problems below this
-
-template <typename T>
-constexpr int ept() {
-  return sizeof(T) == 4 ? kEPT32 : kEPT64;
-}
 
 // row stride rounded up to 128 bytes
 template <typename T>
@@ -237,15 +229,10 @@ struct line_mul<Op, std::void_t<decltype(Op::kLineMul)>> {
   static constexpr int value = Op::kLineMul;
 };
 
-// LDS of a strided tile of `tile` elements (N positions x its lines; the
-// kernel touches only the padded tile after the N twiddles)
-template <typename T, int DIR, int E, int KT, class Op, bool GEN = false>
-int launch_strided_tile(Op& op, int N, size_t tile_max, long long blocks, int nfb,
-                        hipStream_t s) {
-  const size_t tile = std::min(tile_max, (size_t)E * KT);
-  // mixed-radix lengths: two tile buffers (gen_fft stages are out of place)
-  const size_t lds = ((GEN ? 2 : 1) * (tile + tile / 32 + 1) + N) * sizeof(cpx<T>);
-  auto kern = k_strided<T, DIR, E, KT, Op, GEN>;
+template <typename T, int DIR, int LOGN, int LOGE, class Op>
+int launch_strided_kernel(Op& op, unsigned threads, size_t lds, long long blocks, int nfb,
+                          hipStream_t s) {
+  auto kern = k_strided<T, DIR, LOGN, LOGE, Op>;
   static size_t lds_set = 0;
   if (lds > kLdsMax) return fail(FSX_ERR_ARG, "pass needs more LDS than a workgroup has");
   if (lds > lds_set) {
@@ -255,40 +242,53 @@ int launch_strided_tile(Op& op, int N, size_t tile_max, long long blocks, int nf
   }
   int rc = tm_pre(s);
   if (rc) return rc;
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)nfb), dim3(KT), lds, s, op);
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)nfb), dim3(threads), lds, s, op);
   FSX_HIP(hipGetLastError());
   return tm_post(s);
 }
 
+// Length-2^LOGN pass: `tile` elements per workgroup, 2^LOGE per thread.
+template <typename T, int DIR, int LOGN, int LOGE, class Op>
+int launch_strided_p2(Op& op, size_t tile, long long blocks, int nfb, hipStream_t s) {
+  const size_t lds =
+      (tile + tile / 32 + 1 + TilePlan<LOGN, LOGE>::NTW) * sizeof(cpx<T>);
+  return launch_strided_kernel<T, DIR, LOGN, LOGE>(op, (unsigned)(tile >> LOGE), lds, blocks,
+                                                   nfb, s);
+}
+
+// Elements per thread of the strided passes: 16 (FP32 passes of one
+// transform per line) or 8 (FP64; passes that keep several transforms of a
+// line in registers).
+template <typename T, class Op>
+constexpr int strided_loge() {
+  return sizeof(T) == 4 && !Op::kMulti ? 4 : 3;
+}
 template <typename T, int DIR, class Op>
 int launch_strided(Op& op, int N, int nouter, int nlines, int nf, const void* tw,
                    hipStream_t s, bool kio = false, int lines_cap = 0) {
-  constexpr int E = ept<T>() / Op::kEptDiv >= 8 ? ept<T>() / Op::kEptDiv : 8;
-  const int tile = E * kThr;
-  if (N > tile) return fail(FSX_ERR_ARG, "transform length exceeds the tile");
+  constexpr int LOGE = strided_loge<T, Op>();
+  constexpr int run = 128 / (int)sizeof(cpx<T>);  // lines of a 128-byte run
+  const int logN = ilog2(N);
+  const bool p2 = is_pow2(N) && N >= 32;
   const int nfb = Op::kFieldPerBlock ? nf : 1;
-  // FP32 transforms whose tile of kThr threads holds short runs per
-  // position run 2 kThr threads per workgroup (twice the lines) when that
-  // tile's LDS fits: the multi-transform z-passes (halved tiles) when runs
-  // are shorter than a 128-byte line, plain passes below 8 lines (measured:
-  // wider plain y-passes at 8 lines are slower)
-  constexpr int KW = 2 * kThr;
-  constexpr int wide_below = Op::kEptDiv > 1 ? (int)(128 / sizeof(cpx<T>)) : 8;
-  // lengths that are not powers of two: mixed-radix stages in LDS, 512-thread
-  // tiles of at most half the size (two buffers)
-  const bool gen = !is_pow2(N);
-  const bool wide_ok = !gen && sizeof(T) == 4 && tile / N < wide_below &&
-                       ((size_t)E * KW + E * KW / 32 + N) * sizeof(cpx<T>) <= kLdsMax;
-  int L = (wide_ok ? E * KW : tile) / N;
-  if (gen) {
+  int L;
+  if (p2) {
+    const int tile = logN <= 8 ? strided_tile<T, 8, Op>() : strided_tile<T>();
+    if (N > tile) return fail(FSX_ERR_ARG, "transform length exceeds the tile");
+    L = tile / N;
+    op.d.nst = 0;
+  } else {
+    // mixed-radix stages in LDS: tiles of half the size (two buffers)
     op.d.nst = gen_factor(N, op.d.rad);
     if (op.d.nst < 0) return fail(FSX_ERR_ARG, "transform length has too many factors");
-    L = (tile / 2) / N;
+    L = (kGenThr << LOGE) / 2 / N;
     if (L < 1) return fail(FSX_ERR_ARG, "transform length exceeds the tile");
-  } else {
-    op.d.nst = 0;
   }
   while (L & (L - 1)) L &= L - 1;  // power of two
+  // fewest lines of a workgroup: a full wave of threads
+  int Lmin = 1;
+  if (p2)
+    while ((N * Lmin) >> LOGE < 64) Lmin *= 2;
   int cap = 1;
   while (cap < nlines) cap <<= 1;
   if (L > cap) L = cap;
@@ -296,16 +296,19 @@ int launch_strided(Op& op, int N, int nouter, int nlines, int nf, const void* tw
     // tuned lines per tile (power of two)
     while (L > lines_cap && L > 1) L >>= 1;
   } else {
+    // 16 lines are enough: runs of 128 bytes in FP32, 256 in FP64 (with 8
+    // lines, 128 bytes, the FP64 passes of 256^3 are 5 % slower), and
+    // smaller tiles overlap better than 64 KiB ones
+    if (p2)
+      while (L > 16 && L > Lmin) L >>= 1;
     // enough workgroups to fill the chip when the problem is small; long
     // transforms keep more lines per tile (measured on the 2D y-passes:
     // at length 2048, 4 lines in 171 workgroups beat 1 line in 683; at
     // length 1024, 1 line in 342 beats 2 in 171)
     const int min_blocks = N >= 2048 ? 128 : kMinBlocks;
-    while (L > 1 && (long long)nfb * nouter * ((nlines + L - 1) / L) < min_blocks) L >>= 1;
+    while (L > Lmin && (long long)nfb * nouter * ((nlines + L - 1) / L) < min_blocks) L >>= 1;
   }
-  const bool wide = wide_ok && L > tile / N;  // a kThr tile cannot hold L lines
   op.d.N = N;
-  op.d.logN = ilog2(N);
   op.d.L = L;
   op.d.logL = ilog2(L);
   op.d.nouter = nouter;
@@ -314,29 +317,40 @@ int launch_strided(Op& op, int N, int nouter, int nlines, int nf, const void* tw
   op.d.tw = reinterpret_cast<const cpx<T>*>(tw);
   // tiles whose runs are shorter than a 128-byte cache line share lines with
   // their neighbours: keep neighbours on one XCD as for K rows
-  op.d.kio = kio || (size_t)L * sizeof(cpx<T>) < 128;
+  op.d.kio = kio || L < run;
   if (nouter <= 0 || nlines <= 0 || nf <= 0) return 0;
   const long long nchunks = (nlines + L - 1) / L;
   const long long blocks = nchunks * nouter;
   if (blocks > 0x7fffffffLL) return fail(FSX_ERR_ARG, "grid too large");
   // elements the op transforms at once: N L, or N L times its line
-  // multiple when that fits a kThr tile
+  // multiple when that fits a tile
   size_t need = (size_t)N * L;
-  if (gen) {
-    // the same test as the op's own (stacked lines fit the kThr tile)
-    if (need * line_mul<Op>::value <= (size_t)E * kThr) need *= line_mul<Op>::value;
-    return launch_strided_tile<T, DIR, E, kThr, Op, true>(op, N, need, blocks, nfb, s);
+  op.d.stack = 0;
+  if constexpr (line_mul<Op>::value > 1) {
+    op.d.stack = op.stack_ok() &&
+                 need * line_mul<Op>::value <=
+                     (p2 ? (size_t)strided_tile<T>() : (size_t)kGenThr << LOGE);
+    if (op.d.stack) need *= line_mul<Op>::value;
   }
-  if (!wide && need * line_mul<Op>::value <= (size_t)E * kThr) need *= line_mul<Op>::value;
-  // 1024-thread tiles are FP32 only (wide_ok): no FP64 instantiation
-  if constexpr (sizeof(T) == 4)
-    if (wide) return launch_strided_tile<T, DIR, E, KW>(op, N, need, blocks, nfb, s);
-  // small problems (few lines per tile): as many threads as the tile needs
-  if ((size_t)E * kThr / 4 >= need)
-    return launch_strided_tile<T, DIR, E, kThr / 4>(op, N, need, blocks, nfb, s);
-  if ((size_t)E * kThr / 2 >= need)
-    return launch_strided_tile<T, DIR, E, kThr / 2>(op, N, need, blocks, nfb, s);
-  return launch_strided_tile<T, DIR, E, kThr>(op, N, need, blocks, nfb, s);
+  if (!p2) {
+    const size_t lds = (2 * (need + need / 32 + 1) + N) * sizeof(cpx<T>);
+    return launch_strided_kernel<T, DIR, 0, LOGE>(op, kGenThr, lds, blocks, nfb, s);
+  }
+  switch (logN) {
+    case 5: return launch_strided_p2<T, DIR, 5, LOGE>(op, need, blocks, nfb, s);
+    case 6: return launch_strided_p2<T, DIR, 6, LOGE>(op, need, blocks, nfb, s);
+    case 7: return launch_strided_p2<T, DIR, 7, LOGE>(op, need, blocks, nfb, s);
+    case 8: return launch_strided_p2<T, DIR, 8, LOGE>(op, need, blocks, nfb, s);
+    case 9: return launch_strided_p2<T, DIR, 9, LOGE>(op, need, blocks, nfb, s);
+    case 10: return launch_strided_p2<T, DIR, 10, LOGE>(op, need, blocks, nfb, s);
+    case 11: return launch_strided_p2<T, DIR, 11, LOGE>(op, need, blocks, nfb, s);
+    case 12: return launch_strided_p2<T, DIR, 12, LOGE>(op, need, blocks, nfb, s);
+    default:
+      if constexpr (sizeof(T) == 4 && !Op::kMulti) {
+        if (logN == 13) return launch_strided_p2<T, DIR, 13, LOGE>(op, need, blocks, nfb, s);
+      }
+      return fail(FSX_ERR_ARG, "transform length exceeds the tile");
+  }
 }
 
 // Row pass of a length nx that is not a power of two (k_xpass_gen).
@@ -344,8 +358,6 @@ template <typename T, class Op>
 int launch_xpass_gen(Op& op, int nx, int nrows, int nf_in, int nf_out, int mx_in,
                      int ld_in, int mx_out, int ld_out, long long ifs, long long ofs,
                      T scl, const void* tw, hipStream_t s) {
-  constexpr int E = ept<T>() / kXPassEptDiv >= 8 ? ept<T>() / kXPassEptDiv : 8;
-  (void)E;
   // two buffers of complex rows in the workgroup's LDS, after the twiddles
   const int tile = (int)((kLdsMax / sizeof(cpx<T>) - (size_t)nx) / 2);
   const int nfm = nf_in > nf_out ? nf_in : nf_out;
@@ -398,7 +410,7 @@ int launch_xpass(Op& op, int nx, int nrows, int nf_in, int nf_out, int mx_in,
   if (!is_pow2(nx) || nx < 4)
     return launch_xpass_gen<T>(op, nx, nrows, nf_in, nf_out, mx_in, ld_in, mx_out, ld_out,
                                ifs, ofs, scl, tw, s);
-  constexpr int E = ept<T>() / kXPassEptDiv >= 8 ? ept<T>() / kXPassEptDiv : 8;
+  constexpr int E = kXPassE;
   const int tile = E * kXThr;
   const int M = nx / 2;
   const int nfm = nf_in > nf_out ? nf_in : nf_out;
@@ -635,6 +647,26 @@ int inverse_to_w2(fsx_plan_s* p, const cpx<T>* kin, long long kfs, int nf,
   return launch_strided<T, +1>(op, p->ny, p->nz, g.mx, nf, p->tw[1], s);
 }
 
+// W1 (nf fields) -> K through the z-pass (3D); only kept modes written.
+template <typename T>
+int forward_z(fsx_plan_s* p, cpx<T>* kout, long long kfs, int nf, bool pruned,
+              hipStream_t s) {
+  const Geo g = geo<T>(p, pruned);
+  OpZFwd<T> op;
+  op.in = W1<T>(p);
+  op.out = kout;
+  op.ifs = g.fs1;
+  op.ofs = kfs;
+  op.ny = p->ny;
+  op.nkx = p->nkx;
+  op.ld1 = g.ld1;
+  op.ym = g.ym;
+  op.zm = g.zm;
+  op.mask = pruned ? p->d_mask : nullptr;
+  note(K_ZFWD, (double)nf * g.ym.nk() * g.mx * (p->nz + g.zm.nk()) * sizeof(cpx<T>));
+  return launch_strided<T, -1>(op, p->nz, g.ym.nk(), g.mx, nf, p->tw[2], s, true);
+}
+
 // W2 (nf fields) -> K through the y and z passes; only kept modes written.
 template <typename T>
 int forward_from_w2(fsx_plan_s* p, cpx<T>* kout, long long kfs, int nf,
@@ -668,19 +700,7 @@ int forward_from_w2(fsx_plan_s* p, cpx<T>* kout, long long kfs, int nf,
     int rc = launch_strided<T, -1>(op, p->ny, p->nz, g.mx, nf, p->tw[1], s);
     if (rc) return rc;
   }
-  OpZFwd<T> op;
-  op.in = W1<T>(p);
-  op.out = kout;
-  op.ifs = g.fs1;
-  op.ofs = kfs;
-  op.ny = p->ny;
-  op.nkx = p->nkx;
-  op.ld1 = g.ld1;
-  op.ym = g.ym;
-  op.zm = g.zm;
-  op.mask = mask;
-  note(K_ZFWD, (double)nf * g.ym.nk() * g.mx * (p->nz + g.zm.nk()) * sizeof(cpx<T>));
-  return launch_strided<T, -1>(op, p->nz, g.ym.nk(), g.mx, nf, p->tw[2], s, true);
+  return forward_z<T>(p, kout, kfs, nf, pruned, s);
 }
 
 template <typename T>
@@ -776,6 +796,69 @@ int do_ns2d(fsx_plan_s* p, const void* rot, void* out, double beta,
   return forward_from_w2<T>(p, reinterpret_cast<cpx<T>*>(out), 0, 1, true, s);
 }
 
+// y- and x-passes of the 3D tendencies on the planes z0 .. z0 + nzc - 1: W1
+// (nin fields) -> y-inverse -> w2 -> rows (products) -> w2 -> y-forward ->
+// W1 (nout fields, over the inputs of these planes).
+template <typename T>
+int ns3d_plane_chunk(fsx_plan_s* p, int z0, int nzc, cpx<T>* w2, int nin, int nout,
+                     unsigned long long* mx, hipStream_t s, int strat) {
+  const Geo g = geo<T>(p, true);
+  const long long fs2 = (long long)nzc * p->ny * g.ld2;
+  cpx<T>* w1 = W1<T>(p) + (long long)z0 * g.ym.nk() * g.ld1;
+  OpYInv3<T> oy;
+  oy.in = w1;
+  oy.out = w2;
+  oy.ifs = g.fs1;
+  oy.ofs = fs2;
+  oy.ny = p->ny;
+  oy.ld1 = g.ld1;
+  oy.ld2 = g.ld2;
+  oy.ym = g.ym;
+  note(K_YINV, (double)nin * nzc * g.mx * (g.ym.nk() + p->ny) * sizeof(cpx<T>));
+  int rc = launch_strided<T, +1>(oy, p->ny, nzc, g.mx, nin, p->tw[1], s);
+  if (rc) return rc;
+  const double npts = (double)p->nx * p->ny * p->nz;
+  const int rows = nzc * p->ny;
+  note(K_XPASS, (double)(nin + nout) * rows * g.mx * sizeof(cpx<T>));
+  if (strat) {
+    XRStrat<T> xr;
+    rc = launch_xrow<T>(p->nx, rows, g.mx, g.ld2, g.mx, g.ld2, fs2, fs2, T(1.0 / npts), w2, w2,
+                        p->tw[0], mx, xr, s);
+    if (rc == 1) {
+      OpXStrat<T, kXThr> ox;
+      ox.in = w2;
+      ox.out = w2;
+      ox.maxima = mx;
+      rc = launch_xpass<T>(ox, p->nx, rows, nin, nout, g.mx, g.ld2, g.mx, g.ld2, fs2, fs2,
+                           T(1.0 / npts), p->tw[0], s);
+    }
+  } else {
+    XRNS3D<T> xr;
+    rc = launch_xrow<T>(p->nx, rows, g.mx, g.ld2, g.mx, g.ld2, fs2, fs2, T(1.0 / npts), w2, w2,
+                        p->tw[0], mx, xr, s);
+    if (rc == 1) {
+      OpXNS3D<T, kXThr> ox;
+      ox.in = w2;
+      ox.out = w2;
+      ox.maxima = mx;
+      rc = launch_xpass<T>(ox, p->nx, rows, nin, nout, g.mx, g.ld2, g.mx, g.ld2, fs2, fs2,
+                           T(1.0 / npts), p->tw[0], s);
+    }
+  }
+  if (rc) return rc;
+  OpYFwd3<T> of;
+  of.in = w2;
+  of.out = w1;
+  of.ifs = fs2;
+  of.ofs = g.fs1;
+  of.ny = p->ny;
+  of.ld1 = g.ld1;
+  of.ld2 = g.ld2;
+  of.ym = g.ym;
+  note(K_YFWD, (double)nout * nzc * g.mx * (g.ym.nk() + p->ny) * sizeof(cpx<T>));
+  return launch_strided<T, -1>(of, p->ny, nzc, g.mx, nout, p->tw[1], s);
+}
+
 // ns3d (strat = 0): z-pass with curl, y-pass, row pass (v x omega, r2c)
 // into W2 fields 0-2.  ns3d.strat (strat = 1): v, omega and b through the
 // z- and y-passes, row pass producing v x omega and v b into W2 fields 0-5.
@@ -806,47 +889,9 @@ int ns3d_front(fsx_plan_s* p, const void* v, int has_f, double fcor,
                    ((nin - 3.0) * g.zm.nk() + (double)nin * p->nz) * sizeof(cpx<T>));
   int rc = launch_strided<T, +1>(op, p->nz, g.ym.nk(), g.mx, nin, p->tw[2], s, true);
   if (rc) return rc;
-  OpYInv3<T> oy;
-  oy.in = W1<T>(p);
-  oy.out = W2<T>(p);
-  oy.ifs = g.fs1;
-  oy.ofs = g.fs2;
-  oy.ny = p->ny;
-  oy.ld1 = g.ld1;
-  oy.ld2 = g.ld2;
-  oy.ym = g.ym;
-  note(K_YINV, (double)nin * p->nz * g.mx * (g.ym.nk() + p->ny) * sizeof(cpx<T>));
-  rc = launch_strided<T, +1>(oy, p->ny, p->nz, g.mx, nin, p->tw[1], s);
-  if (rc) return rc;
   unsigned long long* mx =
       want_maxima ? reinterpret_cast<unsigned long long*>(p->d_scal) : nullptr;
-  const double npts = (double)p->nx * p->ny * p->nz;
-  note(K_XPASS, (double)(nin + nout) * nrows(p) * g.mx * sizeof(cpx<T>));
-  if (strat) {
-    XRStrat<T> xr;
-    rc = launch_xrow<T>(p->nx, nrows(p), g.mx, g.ld2, g.mx, g.ld2, g.fs2, g.fs2,
-                        T(1.0 / npts), W2<T>(p), W2<T>(p), p->tw[0], mx, xr, s);
-    if (rc != 1) return rc;
-  } else {
-    XRNS3D<T> xr;
-    rc = launch_xrow<T>(p->nx, nrows(p), g.mx, g.ld2, g.mx, g.ld2, g.fs2, g.fs2,
-                        T(1.0 / npts), W2<T>(p), W2<T>(p), p->tw[0], mx, xr, s);
-    if (rc != 1) return rc;
-  }
-  if (strat) {
-    OpXStrat<T, kXThr> ox;
-    ox.in = W2<T>(p);
-    ox.out = W2<T>(p);
-    ox.maxima = mx;
-    return launch_xpass<T>(ox, p->nx, nrows(p), nin, nout, g.mx, g.ld2, g.mx,
-                           g.ld2, g.fs2, g.fs2, T(1.0 / npts), p->tw[0], s);
-  }
-  OpXNS3D<T, kXThr> ox;
-  ox.in = W2<T>(p);
-  ox.out = W2<T>(p);
-  ox.maxima = mx;
-  return launch_xpass<T>(ox, p->nx, nrows(p), nin, nout, g.mx, g.ld2, g.mx,
-                         g.ld2, g.fs2, g.fs2, T(1.0 / npts), p->tw[0], s);
+  return ns3d_plane_chunk<T>(p, 0, p->nz, W2<T>(p), nin, nout, mx, s, strat);
 }
 
 template <typename T>
@@ -854,8 +899,7 @@ int do_ns3d(fsx_plan_s* p, const void* v, void* out, int has_f, double fcor,
             int want_maxima, hipStream_t s) {
   int rc = ns3d_front<T>(p, v, has_f, fcor, want_maxima, s);
   if (rc) return rc;
-  return forward_from_w2<T>(p, reinterpret_cast<cpx<T>*>(out),
-                            (long long)kelems(p), 3, true, s);
+  return forward_z<T>(p, reinterpret_cast<cpx<T>*>(out), (long long)kelems(p), 3, true, s);
 }
 
 template <typename T>
@@ -1095,20 +1139,6 @@ int do_ns3d_rk(fsx_plan_s* p, int scheme, int stage, void* S, void* tmp,
   rc = ns3d_front<T>(p, stage == 0 ? S : t1, has_f, fcor, use_cfl, s);
   if (rc) return rc;
   const Geo g = geo<T>(p, true);
-  {
-    OpYFwd3<T> op;
-    op.in = W2<T>(p);
-    op.out = W1<T>(p);
-    op.ifs = g.fs2;
-    op.ofs = g.fs1;
-    op.ny = p->ny;
-    op.ld1 = g.ld1;
-    op.ld2 = g.ld2;
-    op.ym = g.ym;
-    note(K_YFWD, 3.0 * p->nz * g.mx * (g.ym.nk() + p->ny) * sizeof(cpx<T>));
-    rc = launch_strided<T, -1>(op, p->ny, p->nz, g.mx, 3, p->tw[1], s);
-    if (rc) return rc;
-  }
   if (use_cfl && (rc = cfl_end(p, 3, cfl, dt_max, s))) return rc;
   if ((rc = forcing_stage0<T>(p, stage, S, s))) return rc;
   OpZFwdRK3<T> op;
@@ -1161,20 +1191,6 @@ int do_strat(fsx_plan_s* p, int scheme, int stage, void* S, void* tmp, void* t1,
   rc = ns3d_front<T>(p, src, has_f, fcor, reduce, s, 1);
   if (rc) return rc;
   const Geo g = geo<T>(p, true);
-  {
-    OpYFwd3<T> op;
-    op.in = W2<T>(p);
-    op.out = W1<T>(p);
-    op.ifs = g.fs2;
-    op.ofs = g.fs1;
-    op.ny = p->ny;
-    op.ld1 = g.ld1;
-    op.ld2 = g.ld2;
-    op.ym = g.ym;
-    note(K_YFWD, 6.0 * p->nz * g.mx * (g.ym.nk() + p->ny) * sizeof(cpx<T>));
-    rc = launch_strided<T, -1>(op, p->ny, p->nz, g.mx, 6, p->tw[1], s);
-    if (rc) return rc;
-  }
   if (use_cfl && (rc = cfl_end(p, 3, cfl, dt_max, s))) return rc;
   if ((rc = forcing_stage0<T>(p, stage, S, s))) return rc;
   OpZFwdRKStrat<T> op;

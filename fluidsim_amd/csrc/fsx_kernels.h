@@ -22,235 +22,9 @@
 
 #include "fsx_fft.h"
 #include "fsx_pointwise.h"
+#include "fsx_tile.h"
 
 namespace fsx {
-
-template <typename T>
-struct StridedDesc {
-  int N, logN;    // FFT length
-  int L, logL;    // lines per tile (power of two)
-  int nouter;     // number of independent planes
-  int nlines;     // lines per plane
-  int nf;         // fields transformed one after the other
-  int kio;        // tiles remapped per XCD (K rows, or runs under a cache line)
-  const cpx<T>* tw;  // exp(-2 pi i m / N), m < N (copied to LDS)
-  // mixed-radix stages of a length that is not a power of two (gen_fft)
-  int nst;
-  int rad[kMaxStages];
-};
-
-// Hook of tile_fft run after the first stage (default: nothing).
-struct NoFetch {
-  __device__ __forceinline__ void operator()(int, int, int) const {}
-};
-
-// Stage plan of tile_fft_p2 for a length 2^logN with EPT elements per
-// thread: log2 of the first stage's radix (0: a single stage of radix
-// 2^logN) and of the last stage's; the stages between are radix 8.  With
-// 16 elements per thread a radix-16 first stage (and a radix-16 last one
-// where four factors are left) replaces a radix-8 stage plus a radix-2 or
-// -4 one wherever logN is not a multiple of 3: one LDS round trip and its
-// two barriers fewer per tile (1024 = 16 8 8, 2048 = 16 8 16, 256 = 16 16).
-template <int EPT>
-__device__ __forceinline__ void tile_plan(int logN, int& lfirst, int& llast) {
-  if (logN <= 3 || (EPT >= 16 && logN == 4)) {
-    lfirst = 0;
-    llast = logN;
-    return;
-  }
-  const bool r16 = EPT >= 16 && logN % 3 != 0;
-  lfirst = r16 ? 4 : 3;
-  const int lmax = r16 ? 4 : 3;
-  int logNs = lfirst;
-  while (logN - logNs > lmax) logNs += 3;
-  llast = logN - logNs;
-}
-
-// Full transform of one tile.  src(e, l, p) gives the input at position p
-// of local line l (e = register slot of the first stage, stable across
-// calls); dst(e, l, p, v) receives the output at position p (e = register
-// slot of the last stage).  fetch(e, l, p) is called for every first-stage
-// slot once that slot's input has been consumed: a multi-transform pass
-// issues there the global loads of its next transform (same slots), so
-// they are in flight during this transform's LDS stages.  Ends with a
-// barrier so buf can be reused.
-template <typename T, int DIR, int EPT, int kT, class Src, class Dst,
-          class Fetch = NoFetch>
-__device__ __forceinline__ void tile_fft_p2(cpx<T>* buf, const cpx<T>* tw,
-                                            int logN, int logL, Src&& src,
-                                            Dst&& dst, const Fetch& fetch = Fetch()) {
-  const int lmask = (1 << logL) - 1;
-  int lfirst, llast;
-  tile_plan<EPT>(logN, lfirst, llast);
-  if (lfirst == 0) {
-    // single stage: HBM -> registers -> HBM
-    auto single = [&](auto Rc) {
-      constexpr int R = decltype(Rc)::value;
-      constexpr int NB = EPT / R;
-#pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        const int b = threadIdx.x + i * kT;
-        if (b <= lmask) {
-          cpx<T> v[R];
-#pragma unroll
-          for (int r = 0; r < R; ++r) v[r] = src(i * R + r, b, r);
-          dftR<T, DIR, R>(v);
-#pragma unroll
-          for (int r = 0; r < R; ++r) dst(i * R + r, b, r, v[r]);
-#pragma unroll
-          for (int r = 0; r < R; ++r) fetch(i * R + r, b, r);
-        }
-      }
-    };
-    if constexpr (EPT >= 16) {
-      if (logN == 4) single(std::integral_constant<int, 16>());
-    }
-    if (logN == 3)
-      single(std::integral_constant<int, 8>());
-    else if (logN == 2)
-      single(std::integral_constant<int, 4>());
-    else if (logN < 2)
-      single(std::integral_constant<int, 2>());
-    __syncthreads();
-    return;
-  }
-  // first stage, Ns = 1: inputs from HBM, outputs to LDS
-  auto first = [&](auto Rc) {
-    constexpr int R = decltype(Rc)::value;
-    constexpr int LOGR = R == 16 ? 4 : 3;
-    constexpr int NB = EPT / R;
-    const int lognb = logN - LOGR;
-    const int total = 1 << (lognb + logL);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int b = threadIdx.x + i * kT;
-      if (b < total) {
-        const int line = b & lmask;
-        const int j = b >> logL;
-        cpx<T> v[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) v[r] = src(i * R + r, line, j + (r << lognb));
-        dftR<T, DIR, R>(v);
-#pragma unroll
-        for (int r = 0; r < R; ++r) buf[lpad((((j << LOGR) + r) << logL) + line)] = v[r];
-#pragma unroll
-        for (int r = 0; r < R; ++r) fetch(i * R + r, line, j + (r << lognb));
-      }
-    }
-    __syncthreads();
-  };
-  if constexpr (EPT >= 16) {
-    if (lfirst == 4) first(std::integral_constant<int, 16>());
-  }
-  if (lfirst == 3) first(std::integral_constant<int, 8>());
-  int logNs = lfirst;
-  while (logN - logNs > llast) {
-    lds_stage_lf<T, DIR, EPT, 8, kT>(buf, logN, logNs, logL, tw);
-    logNs += 3;
-  }
-  // last stage: k = j, outputs at j + r Ns, to HBM
-  auto last = [&](auto Rc) {
-    constexpr int R = decltype(Rc)::value;
-    constexpr int LOGR = R == 16 ? 4 : (R == 8 ? 3 : (R == 4 ? 2 : 1));
-    constexpr int NB = EPT / R;
-    const int lognb = logN - LOGR;
-    const int total = 1 << (lognb + logL);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int b = threadIdx.x + i * kT;
-      if (b < total) {
-        const int line = b & lmask;
-        const int j = b >> logL;
-        cpx<T> v[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) v[r] = buf[lpad(((j + (r << lognb)) << logL) + line)];
-        twiddle<T, DIR, R, LOGR>(v, j, logN, logN - LOGR, tw, 0);
-        dftR<T, DIR, R>(v);
-#pragma unroll
-        for (int r = 0; r < R; ++r) dst(i * R + r, line, j + (r << lognb), v[r]);
-      }
-    }
-  };
-  if constexpr (EPT >= 16) {
-    if (llast == 4) last(std::integral_constant<int, 16>());
-  }
-  if (llast == 3)
-    last(std::integral_constant<int, 8>());
-  else if (llast == 2)
-    last(std::integral_constant<int, 4>());
-  else if (llast == 1)
-    last(std::integral_constant<int, 2>());
-  __syncthreads();
-}
-
-// Full transform of one tile of 2^logL lines of length d.N.  GEN = false:
-// power-of-two length (tile_fft_p2, registers at both ends).  GEN = true:
-// any length (gen_fft); slot e of both src and dst is the tile element
-// threadIdx.x + e kT (line-fast), and the tile uses two LDS buffers.
-template <typename T, int DIR, int EPT, int kT, bool GEN, class Src, class Dst,
-          class Fetch = NoFetch>
-__device__ __forceinline__ void tile_fft(cpx<T>* buf, const cpx<T>* tw,
-                                         const StridedDesc<T>& d, int logL, Src&& src,
-                                         Dst&& dst, const Fetch& fetch = Fetch()) {
-  if constexpr (!GEN) {
-    tile_fft_p2<T, DIR, EPT, kT>(buf, tw, d.logN, logL, src, dst, fetch);
-  } else {
-    const int tot = d.N << logL;
-    const int lmask = (1 << logL) - 1;
-    cpx<T>* A = buf;
-    cpx<T>* B = buf + tot + (tot >> 5) + 1;
-    const TileLayout lay{logL, 0};
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      const int idx = threadIdx.x + e * kT;
-      if (idx < tot) A[lpad(idx)] = src(e, idx & lmask, idx >> logL);
-    }
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      const int idx = threadIdx.x + e * kT;
-      if (idx < tot) fetch(e, idx & lmask, idx >> logL);
-    }
-    __syncthreads();
-    const cpx<T>* res = gen_fft<T, DIR, kT>(A, B, lay, tw, d.N, 1 << logL, d.nst, d.rad);
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      const int idx = threadIdx.x + e * kT;
-      if (idx < tot) dst(e, idx & lmask, idx >> logL, res[lpad(idx)]);
-    }
-    __syncthreads();
-  }
-}
-
-// Position of register slot e of tile_fft's last stage: returns false when
-// the slot holds no butterfly output, else its local line and position.
-template <int EPT, int kT, bool GEN, typename T>
-__device__ __forceinline__ bool last_slot(int e, const StridedDesc<T>& d, int logL,
-                                          int& line, int& p) {
-  if constexpr (GEN) {
-    const int idx = threadIdx.x + e * kT;
-    if (idx >= (d.N << logL)) return false;
-    line = idx & ((1 << logL) - 1);
-    p = idx >> logL;
-    return true;
-  }
-  const int logN = d.logN;
-  int lfirst, logR;
-  tile_plan<EPT>(logN, lfirst, logR);
-  const int i = e >> logR, r = e & ((1 << logR) - 1);
-  if (i >= (EPT >> logR)) return false;
-  const int b = threadIdx.x + i * kT;
-  const int lognb = logN - logR;
-  if (b >= (1 << (lognb + logL))) return false;
-  line = b & ((1 << logL) - 1);
-  p = (b >> logL) + (r << lognb);
-  return true;
-}
-
-// Elements per thread of the multi-transform z-passes (tile = kThr x EPT /
-// div): the curl pass stashes 3 and the Runge-Kutta passes 3-4 transforms
-// in registers, so their tiles are halved by default.
-constexpr int kZCurlEptDiv = 2;
-constexpr int kZRKEptDiv = 2;
 
 // ---------------------------------------------------------------- strided
 // Workgroups are dispatched round-robin over the XCDs (workgroup b runs on
@@ -268,40 +42,50 @@ __device__ __forceinline__ int xcd_remap(int b, int nb) {
   return x < rem ? x * (q + 1) + local : rem * (q + 1) + (x - rem) * q + local;
 }
 
-template <typename T, int DIR, int EPT, int kT, class Op, bool GEN = false>
-static __global__ __launch_bounds__(kT) void k_strided(Op op) {
+// Strided pass.  LOGN > 0: length 2^LOGN, N L / 2^LOGE threads (4 L where
+// the op stacks its outputs); LOGN = 0: any length, kGenThr threads.
+template <typename T, int DIR, int LOGN, int LOGE, class Op>
+static __global__ __launch_bounds__((LOGN > 0 ? strided_tile<T, LOGN, Op>() >> LOGE : kGenThr))
+void k_strided(Op op) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const StridedDesc<T>& d = op.d;
   cpx<T>* s_tw = reinterpret_cast<cpx<T>*>(smem_raw);
-  cpx<T>* buf = s_tw + d.N;
-  for (int i = threadIdx.x; i < d.N; i += kT) s_tw[i] = d.tw[i];
+  cpx<T>* buf;
   // (tile_fft's first barrier precedes every twiddle read)
+  if constexpr (LOGN > 0) {
+    buf = s_tw + TilePlan<LOGN, LOGE>::NTW;
+    tile_twiddles<T, LOGN, LOGE>(s_tw, d.tw);
+  } else {
+    buf = s_tw + d.N;
+    for (int i = threadIdx.x; i < d.N; i += kGenThr) s_tw[i] = d.tw[i];
+  }
   const int nchunks = (d.nlines + d.L - 1) >> d.logL;
   const int b = d.kio ? xcd_remap(blockIdx.x, gridDim.x) : (int)blockIdx.x;
   const int o = b / nchunks;
   const int line0 = (b - o * nchunks) << d.logL;
-  op.template run<DIR, EPT, kT, GEN>(buf, s_tw, o, line0);
+  op.template run<DIR, LOGN, LOGE>(buf, s_tw, o, line0);
 }
 
-// Plain pass: one field per workgroup (blockIdx.y), load()/store().
+// Plain pass: one field per workgroup (blockIdx.y).  The op names the two
+// sides of field f, plane o: geometry (in_lines, out_lines) and base
+// pointers of line line0 (in_base, out_base).
 template <typename T, class Self>
 struct PlainRun {
-  static constexpr int kEptDiv = 1;
+  static constexpr bool kMulti = false;
   static constexpr bool kFieldPerBlock = true;
-  template <int DIR, int EPT, int kT, bool GEN>
+  template <int DIR, int LOGN, int LOGE>
   __device__ __forceinline__ void run(cpx<T>* buf, const cpx<T>* tw, int o, int line0) const {
     const Self& s = static_cast<const Self&>(*this);
-    const int nlines = s.d.nlines;
-    const int f = blockIdx.y;
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, s.d, s.d.logL,
-        [&](int, int l, int p) {
-          const int line = line0 + l;
-          return line < nlines ? s.load(f, o, line, p) : zero<T>();
-        },
-        [&](int, int l, int p, cpx<T> v) {
-          const int line = line0 + l;
-          if (line < nlines) s.store(f, o, line, p, v);
+    const int nl = s.d.nlines - line0, f = blockIdx.y;
+    const Lines gi = s.in_lines(nl), go = s.out_lines(nl);
+    const cpx<T>* in = s.in + f * s.ifs + s.in_plane(o) + line0;
+    cpx<T>* out = s.out + f * s.ofs + s.out_plane(o) + line0;
+    const unsigned char* mask = s.mask ? s.mask + s.out_plane(o) + line0 : nullptr;
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, s.d, s.d.logL, [&](const Slot& t) { return ln_load<LOGN, T>(gi, in, t); },
+        [&](const Slot& t, cpx<T> v) {
+          if (ln_masked<LOGN>(go, mask, t)) v = zero<T>();
+          ln_store<LOGN, T>(go, out, t, v);
         });
   }
 };
@@ -316,13 +100,15 @@ struct OpZInv : PlainRun<T, OpZInv<T>> {
   long long ifs, ofs;  // field strides (elements)
   int ny, nkx, ld1;
   AxisMap ym, zm;
-  __device__ cpx<T> load(int f, int o, int l, int p) const {
-    if (zm.compact(p) < 0) return zero<T>();
-    return in[f * ifs + (p * ny + ym.full(o)) * nkx + l];
+  static constexpr const unsigned char* mask = nullptr;
+  __device__ Lines in_lines(int nl) const {
+    return lines_of((unsigned)ny * (unsigned)nkx, zm, false, nl);
   }
-  __device__ void store(int f, int o, int l, int p, cpx<T> v) const {
-    out[f * ofs + (p * ym.nk() + o) * ld1 + l] = v;
+  __device__ Lines out_lines(int nl) const {
+    return lines_all((unsigned)ym.nk() * (unsigned)ld1, zm.n, nl);
   }
+  __device__ long long in_plane(int o) const { return (long long)ym.full(o) * nkx; }
+  __device__ long long out_plane(int o) const { return (long long)o * ld1; }
 };
 
 // y-pass, inverse: W1 (nz, nyk, ld1) -> W2 (nz, ny, ld2); planes are z.
@@ -334,14 +120,11 @@ struct OpYInv3 : PlainRun<T, OpYInv3<T>> {
   long long ifs, ofs;
   int ny, ld1, ld2;
   AxisMap ym;
-  __device__ cpx<T> load(int f, int z, int l, int p) const {
-    const int jy = ym.compact(p);
-    if (jy < 0) return zero<T>();
-    return in[f * ifs + (z * ym.nk() + jy) * ld1 + l];
-  }
-  __device__ void store(int f, int z, int l, int p, cpx<T> v) const {
-    out[f * ofs + (z * ny + p) * ld2 + l] = v;
-  }
+  static constexpr const unsigned char* mask = nullptr;
+  __device__ Lines in_lines(int nl) const { return lines_of(ld1, ym, true, nl); }
+  __device__ Lines out_lines(int nl) const { return lines_all(ld2, ny, nl); }
+  __device__ long long in_plane(int z) const { return (long long)z * ym.nk() * ld1; }
+  __device__ long long out_plane(int z) const { return (long long)z * ny * ld2; }
 };
 
 // y-pass, forward: W2 (nz, ny, ld2) -> W1 (nz, nyk, ld1).
@@ -353,13 +136,11 @@ struct OpYFwd3 : PlainRun<T, OpYFwd3<T>> {
   long long ifs, ofs;
   int ny, ld1, ld2;
   AxisMap ym;
-  __device__ cpx<T> load(int f, int z, int l, int p) const {
-    return in[f * ifs + (z * ny + p) * ld2 + l];
-  }
-  __device__ void store(int f, int z, int l, int p, cpx<T> v) const {
-    const int jy = ym.compact(p);
-    if (jy >= 0) out[f * ofs + (z * ym.nk() + jy) * ld1 + l] = v;
-  }
+  static constexpr const unsigned char* mask = nullptr;
+  __device__ Lines in_lines(int nl) const { return lines_all(ld2, ny, nl); }
+  __device__ Lines out_lines(int nl) const { return lines_of(ld1, ym, true, nl); }
+  __device__ long long in_plane(int z) const { return (long long)z * ny * ld2; }
+  __device__ long long out_plane(int z) const { return (long long)z * ym.nk() * ld1; }
 };
 
 // z-pass, forward: W1 (nz, nyk, ld1) -> K (nz, ny, nkx); only kept modes
@@ -373,15 +154,14 @@ struct OpZFwd : PlainRun<T, OpZFwd<T>> {
   int ny, nkx, ld1;
   AxisMap ym, zm;
   const unsigned char* mask;
-  __device__ cpx<T> load(int f, int jy, int l, int p) const {
-    return in[f * ifs + (p * ym.nk() + jy) * ld1 + l];
+  __device__ Lines in_lines(int nl) const {
+    return lines_all((unsigned)ym.nk() * (unsigned)ld1, zm.n, nl);
   }
-  __device__ void store(int f, int jy, int l, int p, cpx<T> v) const {
-    if (zm.compact(p) < 0) return;
-    const int idx = (p * ny + ym.full(jy)) * nkx + l;
-    if (mask && mask[idx]) v = zero<T>();
-    out[f * ofs + idx] = v;
+  __device__ Lines out_lines(int nl) const {
+    return lines_of((unsigned)ny * (unsigned)nkx, zm, false, nl);
   }
+  __device__ long long in_plane(int o) const { return (long long)o * ld1; }
+  __device__ long long out_plane(int o) const { return (long long)ym.full(o) * nkx; }
 };
 
 // 2D y-pass, inverse: K (ny, nkx) -> W2 (ny, ld2).
@@ -393,13 +173,11 @@ struct OpYInv2 : PlainRun<T, OpYInv2<T>> {
   long long ifs, ofs;
   int nkx, ld2;
   AxisMap ym;
-  __device__ cpx<T> load(int f, int, int l, int p) const {
-    if (ym.compact(p) < 0) return zero<T>();
-    return in[f * ifs + p * nkx + l];
-  }
-  __device__ void store(int f, int, int l, int p, cpx<T> v) const {
-    out[f * ofs + p * ld2 + l] = v;
-  }
+  static constexpr const unsigned char* mask = nullptr;
+  __device__ Lines in_lines(int nl) const { return lines_of(nkx, ym, false, nl); }
+  __device__ Lines out_lines(int nl) const { return lines_all(ld2, ym.n, nl); }
+  __device__ long long in_plane(int) const { return 0; }
+  __device__ long long out_plane(int) const { return 0; }
 };
 
 // 2D y-pass, forward: W2 (ny, ld2) -> K (ny, nkx), kept modes only.
@@ -412,15 +190,10 @@ struct OpYFwd2 : PlainRun<T, OpYFwd2<T>> {
   int nkx, ld2;
   AxisMap ym;
   const unsigned char* mask;
-  __device__ cpx<T> load(int f, int, int l, int p) const {
-    return in[f * ifs + p * ld2 + l];
-  }
-  __device__ void store(int f, int, int l, int p, cpx<T> v) const {
-    if (ym.compact(p) < 0) return;
-    const int idx = p * nkx + l;
-    if (mask && mask[idx]) v = zero<T>();
-    out[f * ofs + idx] = v;
-  }
+  __device__ Lines in_lines(int nl) const { return lines_all(ld2, ym.n, nl); }
+  __device__ Lines out_lines(int nl) const { return lines_of(nkx, ym, false, nl); }
+  __device__ long long in_plane(int) const { return 0; }
+  __device__ long long out_plane(int) const { return 0; }
 };
 
 // ns3d z-pass, inverse, with the curl folded in.  omega = i k x v needs
@@ -432,7 +205,7 @@ struct OpYFwd2 : PlainRun<T, OpYFwd2<T>> {
 // each input read from HBM once; outputs 0-2 are v, 3-5 omega.
 template <typename T>
 struct OpZInvCurl {
-  static constexpr int kEptDiv = kZCurlEptDiv;  // register stashes: half-size tiles
+  static constexpr bool kMulti = true;  // register stashes: half-size tiles
   static constexpr bool kFieldPerBlock = false;
   StridedDesc<T> d;
   const cpx<T>* in;  // 3 fields
@@ -445,75 +218,67 @@ struct OpZInvCurl {
   T fcor;
   int with_b;  // ns3d.strat: input 3 (b) transformed into output 6
 
-  template <int DIR, int EPT, int kT, bool GEN>
+  template <int DIR, int LOGN, int LOGE>
   __device__ __forceinline__ void run(cpx<T>* buf, const cpx<T>* tw, int o, int line0) const {
-    const int nlines = d.nlines;
+    constexpr int E = 1 << LOGE;
+    const int nl = d.nlines - line0;
     const int iy = ym.full(o);
     const T ky = T(ksigned(iy, ny)) * dky;
-    const int nyk = ym.nk();
-    cpx<T> sVz[EPT], sv[EPT], sVy[EPT];
-    auto ld = [&](int c, int l, int p) {
-      const int line = line0 + l;
-      if (line >= nlines || zm.compact(p) < 0) return zero<T>();
-      return in[c * ifs + (p * ny + iy) * nkx + line];
-    };
-    auto st = [&](int c, int l, int p, cpx<T> v) {
-      const int line = line0 + l;
-      if (line < nlines) out[c * ofs + (p * nyk + o) * ld1 + line] = v;
-    };
-    auto kz_of = [&](int p) { return T(ksigned(p, nz)) * dkz; };
+    const Lines gi = lines_of((unsigned)ny * (unsigned)nkx, zm, false, nl);
+    const Lines go = lines_all((unsigned)ym.nk() * (unsigned)ld1, nz, nl);
+    const cpx<T>* in0 = in + (long long)iy * nkx + line0;
+    cpx<T>* out0 = out + (long long)o * ld1 + line0;
+    cpx<T> sVz[E], sv[E], sVy[E];
+    auto ld = [&](int c, const Slot& t) { return ln_load<LOGN, T>(gi, in0 + c * ifs, t); };
+    auto st = [&](int c, const Slot& t, cpx<T> v) { ln_store<LOGN, T>(go, out0 + c * ofs, t, v); };
+    auto kz_of = [&](const Slot& t) { return T(ksigned(t.pos(), nz)) * dkz; };
+    auto kx_of = [&](const Slot& t) { return T(line0 + t.line) * dkx; };
     // Each input is loaded once, into sv (vy, then vx) or sVz (b, once Vz
     // is no longer needed), while the transform before the one that first
     // uses it runs (tile_fft's fetch hook): only the first load of a tile
     // waits for HBM.
     // Vz; vy fetched
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL, [&](int, int l, int p) { return ld(2, l, p); },
-        [&](int e, int l, int p, cpx<T> v) {
-          sVz[e] = v;
-          st(2, l, p, v);
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, d, d.logL, [&](const Slot& t) { return ld(2, t); },
+        [&](const Slot& t, cpx<T> v) {
+          sVz[t.e] = v;
+          st(2, t, v);
         },
-        [&](int e, int l, int p) { sv[e] = ld(1, l, p); });
+        [&](const Slot& t) { sv[t.e] = ld(1, t); });
     // omega_x = i ky Vz - Dz[vy]
-    tile_fft<T, DIR, EPT, kT, GEN>(
+    tile_fft<T, DIR, LOGN, LOGE>(
         buf, tw, d, d.logL,
-        [&](int e, int, int p) { return mul_i(scale(sv[e], kz_of(p))); },
-        [&](int e, int l, int p, cpx<T> v) {
-          st(3, l, p, mul_i(scale(sVz[e], ky)) - v);
-        });
+        [&](const Slot& t) { return mul_i(scale(sv[t.e], kz_of(t))); },
+        [&](const Slot& t, cpx<T> v) { st(3, t, mul_i(scale(sVz[t.e], ky)) - v); });
     // Vy; vx fetched over vy once the first stage has read it
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL, [&](int e, int, int) { return sv[e]; },
-        [&](int e, int l, int p, cpx<T> v) {
-          sVy[e] = v;
-          st(1, l, p, v);
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, d, d.logL, [&](const Slot& t) { return sv[t.e]; },
+        [&](const Slot& t, cpx<T> v) {
+          sVy[t.e] = v;
+          st(1, t, v);
         },
-        [&](int e, int l, int p) { sv[e] = ld(0, l, p); });
+        [&](const Slot& t) { sv[t.e] = ld(0, t); });
     // omega_y = Dz[vx] - i kx Vz
-    tile_fft<T, DIR, EPT, kT, GEN>(
+    tile_fft<T, DIR, LOGN, LOGE>(
         buf, tw, d, d.logL,
-        [&](int e, int, int p) { return mul_i(scale(sv[e], kz_of(p))); },
-        [&](int e, int l, int p, cpx<T> v) {
-          const T kx = T(line0 + l) * dkx;
-          st(4, l, p, v - mul_i(scale(sVz[e], kx)));
-        });
+        [&](const Slot& t) { return mul_i(scale(sv[t.e], kz_of(t))); },
+        [&](const Slot& t, cpx<T> v) { st(4, t, v - mul_i(scale(sVz[t.e], kx_of(t)))); });
     // Vx and omega_z = i kx Vy - i ky Vx (+ f); b fetched into sVz
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL, [&](int e, int, int) { return sv[e]; },
-        [&](int e, int l, int p, cpx<T> v) {
-          const T kx = T(line0 + l) * dkx;
-          st(0, l, p, v);
-          cpx<T> w = mul_i(scale(sVy[e], kx) - scale(v, ky));
-          if (has_f && iy == 0 && line0 + l == 0) w.x += fcor;
-          st(5, l, p, w);
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, d, d.logL, [&](const Slot& t) { return sv[t.e]; },
+        [&](const Slot& t, cpx<T> v) {
+          st(0, t, v);
+          cpx<T> w = mul_i(scale(sVy[t.e], kx_of(t)) - scale(v, ky));
+          if (has_f && iy == 0 && line0 + t.line == 0) w.x += fcor;
+          st(5, t, w);
         },
-        [&](int e, int l, int p) {
-          if (with_b) sVz[e] = ld(3, l, p);
+        [&](const Slot& t) {
+          if (with_b) sVz[t.e] = ld(3, t);
         });
     if (with_b)
-      tile_fft<T, DIR, EPT, kT, GEN>(
-          buf, tw, d, d.logL, [&](int e, int, int) { return sVz[e]; },
-          [&](int, int l, int p, cpx<T> v) { st(6, l, p, v); });
+      tile_fft<T, DIR, LOGN, LOGE>(
+          buf, tw, d, d.logL, [&](const Slot& t) { return sVz[t.e]; },
+          [&](const Slot& t, cpx<T> v) { st(6, t, v); });
   }
 };
 
@@ -522,10 +287,12 @@ struct OpZInvCurl {
 // d_y rot = i ky rot (k^2 = 1e-14 at k = 0, the K2_not0 convention).
 template <typename T>
 struct OpYInv2NS {
-  static constexpr int kEptDiv = 1;
+  static constexpr bool kMulti = false;
   static constexpr bool kFieldPerBlock = false;
   // the four outputs can share one tile as 4 L lines (small transforms)
   static constexpr int kLineMul = 4;
+  // whether the stacked outputs are in reach of a 32-bit offset
+  bool stack_ok() const { return (4.0 * ofs) * sizeof(cpx<T>) < kBufMax; }
   StridedDesc<T> d;
   const cpx<T>* in;
   cpx<T>* out;
@@ -536,73 +303,65 @@ struct OpYInv2NS {
   AxisMap ym;
   T dkx, dky;
 
-  template <int DIR, int EPT, int kT, bool GEN>
+  // multiplier (without i) of output c at (line, p)
+  __device__ __forceinline__ T factor(int c, int line, int p) const {
+    const T kx = T(line) * dkx, ky = T(ksigned(p, ny)) * dky;
+    if (c >= 2) return c == 2 ? kx : ky;
+    T k2 = fma_t(kx, kx, ky * ky);
+    if (k2 == T(0)) k2 = T(1e-14);
+    return (c == 0 ? ky : -kx) * (T(1) / k2);
+  }
+
+  template <int DIR, int LOGN, int LOGE>
   __device__ __forceinline__ void run(cpx<T>* buf, const cpx<T>* tw, int o, int line0) const {
-    const int nlines = d.nlines;
-    const cpx<T>* in = this->in + o * ips;
-    cpx<T>* out = this->out + o * ops;
-    cpx<T> sr[EPT];
-    auto st = [&](int c, int l, int p, cpx<T> v) {
-      const int line = line0 + l;
-      if (line < nlines) out[c * ofs + p * ld2 + line] = v;
-    };
-    auto inv_k2 = [&](int l, int p) {
-      const T kx = T(line0 + l) * dkx, ky = T(ksigned(p, ny)) * dky;
-      T k2 = kx * kx + ky * ky;
-      if (k2 == T(0)) k2 = T(1e-14);
-      return T(1) / k2;
-    };
-    if (((size_t)d.N << (d.logL + 2)) <= (size_t)EPT * kT) {
+    constexpr int E = 1 << LOGE;
+    const int nl = d.nlines - line0;
+    const Lines gi = lines_of(nkx, ym, false, nl), go = lines_all(ld2, ny, nl);
+    const cpx<T>* in0 = in + o * ips + line0;
+    cpx<T>* out0 = out + o * ops + line0;
+    if (d.stack) {
       // one transform of 4 L lines: line l is output l >> logL of line
       // l & (L - 1), each line computed as in the sequential form below
       const int lm = (1 << d.logL) - 1;
-      tile_fft<T, DIR, EPT, kT, GEN>(
+      tile_fft<T, DIR, LOGN, LOGE>(
           buf, tw, d, d.logL + 2,
-          [&](int, int l, int p) {
-            const int c = l >> d.logL, li = l & lm;
-            const int line = line0 + li;
-            cpx<T> r = zero<T>();
-            if (line < nlines && ym.compact(p) >= 0) r = in[p * nkx + line];
-            T f;
-            if (c == 0)
-              f = T(ksigned(p, ny)) * dky * inv_k2(li, p);
-            else if (c == 1)
-              f = -(T(line0 + li) * dkx) * inv_k2(li, p);
-            else if (c == 2)
-              f = T(line0 + li) * dkx;
-            else
-              f = T(ksigned(p, ny)) * dky;
-            return mul_i(scale(r, f));
+          [&](const Slot& t) {
+            const Slot u{t.e, t.line & lm, t.j, t.pr};
+            const cpx<T> r = ln_load<LOGN, T>(gi, in0, u);
+            return mul_i(scale(r, factor(t.line >> d.logL, line0 + u.line, t.pos())));
           },
-          [&](int, int l, int p, cpx<T> v) { st(l >> d.logL, l & lm, p, v); });
+          [&](const Slot& t, cpx<T> v) {
+            const Slot u{t.e, t.line & lm, t.j, t.pr};
+            const int c = t.line >> d.logL;
+            if constexpr (LOGN > 0) {
+              // the output field is part of the lane's offset (the launcher
+              // stacks only where it fits 32 bits)
+              const unsigned off = ((unsigned)u.j * go.ps + (unsigned)u.line +
+                                    (unsigned)c * (unsigned)ofs) * (unsigned)sizeof(cpx<T>);
+              buf_store<T>(buf_rsrc(out0 + ln_base<LOGN>(go, u), kBufMax),
+                           ln_kept<LOGN>(go, u) ? off : kOOB, v);
+            } else {
+              ln_store<LOGN, T>(go, out0 + c * ofs, u, v);
+            }
+          });
       return;
     }
-    tile_fft<T, DIR, EPT, kT, GEN>(
+    cpx<T> sr[E];
+    tile_fft<T, DIR, LOGN, LOGE>(
         buf, tw, d, d.logL,
-        [&](int e, int l, int p) {
-          const int line = line0 + l;
-          cpx<T> r = zero<T>();
-          if (line < nlines && ym.compact(p) >= 0) r = in[p * nkx + line];
-          sr[e] = r;
-          const T ky = T(ksigned(p, ny)) * dky;
-          return mul_i(scale(r, ky * inv_k2(l, p)));
+        [&](const Slot& t) {
+          sr[t.e] = ln_load<LOGN, T>(gi, in0, t);
+          return mul_i(scale(sr[t.e], factor(0, line0 + t.line, t.pos())));
         },
-        [&](int, int l, int p, cpx<T> v) { st(0, l, p, v); });
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL,
-        [&](int e, int l, int p) {
-          const T kx = T(line0 + l) * dkx;
-          return mul_i(scale(sr[e], -kx * inv_k2(l, p)));
-        },
-        [&](int, int l, int p, cpx<T> v) { st(1, l, p, v); });
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL,
-        [&](int e, int l, int) { return mul_i(scale(sr[e], T(line0 + l) * dkx)); },
-        [&](int, int l, int p, cpx<T> v) { st(2, l, p, v); });
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL,
-        [&](int e, int, int p) { return mul_i(scale(sr[e], T(ksigned(p, ny)) * dky)); },
-        [&](int, int l, int p, cpx<T> v) { st(3, l, p, v); });
+        [&](const Slot& t, cpx<T> v) { ln_store<LOGN, T>(go, out0, t, v); });
+#pragma unroll
+    for (int c = 1; c < 4; ++c)
+      tile_fft<T, DIR, LOGN, LOGE>(
+          buf, tw, d, d.logL,
+          [&](const Slot& t) {
+            return mul_i(scale(sr[t.e], factor(c, line0 + t.line, t.pos())));
+          },
+          [&](const Slot& t, cpx<T> v) { ln_store<LOGN, T>(go, out0 + c * ofs, t, v); });
   }
 };
 
@@ -614,35 +373,81 @@ struct OpYInv2NSOne : OpYInv2NS<T> {
   static constexpr bool kFieldPerBlock = true;
   static constexpr int kLineMul = 1;
 
-  template <int DIR, int EPT, int kT, bool GEN>
+  template <int DIR, int LOGN, int LOGE>
   __device__ __forceinline__ void run(cpx<T>* buf, const cpx<T>* tw, int o, int line0) const {
     const StridedDesc<T>& d = this->d;
-    const int nlines = d.nlines;
+    const int nl = d.nlines - line0;
     const int c = blockIdx.y;
-    const cpx<T>* in = this->in + o * this->ips;
-    cpx<T>* out = this->out + o * this->ops + c * this->ofs;
-    const int ny = this->ny, nkx = this->nkx, ld2 = this->ld2;
-    const T dkx = this->dkx, dky = this->dky;
-    tile_fft<T, DIR, EPT, kT, GEN>(
+    const Lines gi = lines_of(this->nkx, this->ym, false, nl);
+    const Lines go = lines_all(this->ld2, this->ny, nl);
+    const cpx<T>* in0 = this->in + o * this->ips + line0;
+    cpx<T>* out0 = this->out + o * this->ops + c * this->ofs + line0;
+    tile_fft<T, DIR, LOGN, LOGE>(
         buf, tw, d, d.logL,
-        [&](int, int l, int p) {
-          const int line = line0 + l;
-          cpx<T> r = zero<T>();
-          if (line < nlines && this->ym.compact(p) >= 0) r = in[p * nkx + line];
-          const T kx = T(line) * dkx, ky = T(ksigned(p, ny)) * dky;
-          T k2 = kx * kx + ky * ky;
-          if (k2 == T(0)) k2 = T(1e-14);
-          const T ik2 = T(1) / k2;
-          // the multipliers of OpYInv2NS's outputs 0..3
-          const T f = c == 0 ? ky * ik2 : (c == 1 ? -kx * ik2 : (c == 2 ? kx : ky));
-          return mul_i(scale(r, f));
+        [&](const Slot& t) {
+          const cpx<T> r = ln_load<LOGN, T>(gi, in0, t);
+          return mul_i(scale(r, this->factor(c, line0 + t.line, t.pos())));
         },
-        [&](int, int l, int p, cpx<T> v) {
-          const int line = line0 + l;
-          if (line < nlines) out[p * ld2 + line] = v;
-        });
+        [&](const Slot& t, cpx<T> v) { ln_store<LOGN, T>(go, out0, t, v); });
   }
 };
+
+// The pass's own argument struct through the kernel-argument pointer, which
+// the optimizer cannot follow back: what is read through it is loaded where
+// it is used, after the transforms, instead of being held in (and spilled
+// from) scalar registers from the start of the kernel.
+template <class Op>
+__device__ __forceinline__ const Op& late_args() {
+  auto* p = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const Op*)(const void*)p;
+}
+
+// Runge-Kutta stage of the modes in a tile's output slots: N(e, n) gives the
+// NV tendencies of slot e (masked here).  The state streams of two
+// slots are loaded before any is used, so that their latencies overlap.
+template <typename T, int NV>
+constexpr int rk_batch() {
+  return NV > 3 ? 1 : 2;
+}
+template <typename T, int NV, int LOGN, int LOGE, class NFn>
+__device__ __forceinline__ void rk_slots(const StridedDesc<T>& d, const Lines& g,
+                                         const RKArgs<T>& rk, const Visc& visc, double dt,
+                                         const unsigned char* mask, long long base, int line0,
+                                         bool along_z, int iky, const NFn& tend) {
+  constexpr int E = 1 << LOGE;
+  constexpr int B = rk_batch<T, NV>();
+#pragma unroll
+  for (int e0 = 0; e0 < E; e0 += B) {
+    std::conditional_t<B == 1, RKDirect<T>, RKStreams<T, NV>> st[B];
+#pragma unroll
+    for (int q = 0; q < B; ++q) {
+      Slot t;
+      if (!last_slot<LOGN, LOGE>(e0 + q, d, d.logL, t)) continue;
+      rk_load(rk, SlotMode<LOGN, T>{g, t, base}, st[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < B; ++q) {
+      Slot t;
+      if (!last_slot<LOGN, LOGE>(e0 + q, d, d.logL, t)) continue;
+      if (B == 1) {
+        // nothing of one slot is kept in registers for the next
+        asm volatile("" : "+v"(t.j), "+v"(t.line));
+      }
+      if (!ln_kept<LOGN>(g, t)) continue;
+      const SlotMode<LOGN, T> m{g, t, base};
+      cpx<T> N[NV];
+      tend(t, m, N);
+      if (ln_masked<LOGN>(g, mask, t)) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) N[v] = zero<T>();
+      }
+      const int kp = ksigned(t.pos(), d.N);
+      rk_point<T, NV>(rk, visc, dt, m, line0 + t.line, along_z ? iky : kp, along_z ? kp : 0, st[q],
+                      N);
+    }
+  }
+}
 
 // ns3d z-pass, forward, with the Runge-Kutta stage folded in: the three
 // tendency components are transformed one after the other (the first two
@@ -650,7 +455,7 @@ struct OpYInv2NSOne : OpYInv2NS<T> {
 // (rk_point); the tendency never goes to HBM.
 template <typename T>
 struct OpZFwdRK3 {
-  static constexpr int kEptDiv = kZRKEptDiv;
+  static constexpr bool kMulti = true;
   static constexpr bool kFieldPerBlock = false;
   StridedDesc<T> d;
   const cpx<T>* in;  // W1, 3 fields
@@ -660,43 +465,41 @@ struct OpZFwdRK3 {
   const unsigned char* mask;
   RKArgs<T> rk;
 
-  template <int DIR, int EPT, int kT, bool GEN>
+  template <int DIR, int LOGN, int LOGE>
   __device__ __forceinline__ void run(cpx<T>* buf, const cpx<T>* tw, int o, int line0) const {
-    const int nlines = d.nlines;
-    const int nyk = ym.nk();
+    constexpr int E = 1 << LOGE;
+    const int nl = d.nlines - line0;
     const int iy = ym.full(o);
-    const int iky = ksigned(iy, ny);
-    const double dt = *rk.dt;
-    cpx<T> s0[EPT], s1[EPT], s2[EPT];
-    auto ld = [&](int c, int l, int p) {
-      const int line = line0 + l;
-      if (line >= nlines) return zero<T>();
-      return in[c * ifs + (p * nyk + o) * ld1 + line];
-    };
+    const Lines gi = lines_all((unsigned)ym.nk() * (unsigned)ld1, d.N, nl);
+    const Lines gk = lines_of((unsigned)ny * (unsigned)nkx, zm, false, nl);
+    const cpx<T>* in0 = in + (long long)o * ld1 + line0;
+    const long long base = (long long)iy * nkx + line0;
+    cpx<T> s0[E], s1[E], s2[E];
+    auto ld = [&](int c, const Slot& t) { return ln_load<LOGN, T>(gi, in0 + c * ifs, t); };
     // input c + 1 is fetched into s(c+1) while transform c runs; the
     // stash's first stage reads it before its last stage stores the output
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL, [&](int, int l, int p) { return ld(0, l, p); },
-        [&](int e, int, int, cpx<T> v) { s0[e] = v; },
-        [&](int e, int l, int p) { s1[e] = ld(1, l, p); });
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL, [&](int e, int, int) { return s1[e]; },
-        [&](int e, int, int, cpx<T> v) { s1[e] = v; },
-        [&](int e, int l, int p) { s2[e] = ld(2, l, p); });
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL, [&](int e, int, int) { return s2[e]; },
-        [&](int e, int, int, cpx<T> v) { s2[e] = v; });
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      int l, p;
-      if (!last_slot<EPT, kT, GEN>(e, d, d.logL, l, p)) continue;
-      const int line = line0 + l;
-      if (line >= nlines || zm.compact(p) < 0) continue;
-      const int idx = (p * ny + iy) * nkx + line;
-      cpx<T> N[3] = {s0[e], s1[e], s2[e]};
-      if (mask && mask[idx]) N[0] = N[1] = N[2] = zero<T>();
-      rk_point<T, 3>(rk, rk.visc, dt, idx, line, iky, ksigned(p, d.N), N);
-    }
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, d, d.logL, [&](const Slot& t) { return ld(0, t); },
+        [&](const Slot& t, cpx<T> v) { s0[t.e] = v; },
+        [&](const Slot& t) { s1[t.e] = ld(1, t); });
+    pin(s0);
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, d, d.logL, [&](const Slot& t) { return s1[t.e]; },
+        [&](const Slot& t, cpx<T> v) { s1[t.e] = v; },
+        [&](const Slot& t) { s2[t.e] = ld(2, t); });
+    pin(s1);
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, d, d.logL, [&](const Slot& t) { return s2[t.e]; },
+        [&](const Slot& t, cpx<T> v) { s2[t.e] = v; });
+    pin(s2);
+    const RKArgs<T>& rk = late_args<OpZFwdRK3>().rk;
+    rk_slots<T, 3, LOGN, LOGE>(d, gk, rk, rk.visc, *rk.dt, mask ? mask + base : nullptr, base,
+                               line0, true, ksigned(iy, ny),
+                               [&](const Slot& t, const SlotMode<LOGN, T>&, cpx<T>* N) {
+                                 N[0] = s0[t.e];
+                                 N[1] = s1[t.e];
+                                 N[2] = s2[t.e];
+                               });
   }
 };
 
@@ -708,7 +511,7 @@ struct OpZFwdRK3 {
 // projection acts on N_v only (rk_point).
 template <typename T>
 struct OpZFwdRKStrat {
-  static constexpr int kEptDiv = kZRKEptDiv;
+  static constexpr bool kMulti = true;
   static constexpr bool kFieldPerBlock = false;
   StridedDesc<T> d;
   const cpx<T>* in;  // W1, 6 fields
@@ -720,66 +523,70 @@ struct OpZFwdRKStrat {
   T N2;
   RKArgs<T> rk;
 
-  template <int DIR, int EPT, int kT, bool GEN>
+  template <int DIR, int LOGN, int LOGE>
   __device__ __forceinline__ void run(cpx<T>* buf, const cpx<T>* tw, int o, int line0) const {
-    const int nlines = d.nlines;
-    const int nyk = ym.nk();
+    constexpr int E = 1 << LOGE;
+    const int nl = d.nlines - line0;
     const int iy = ym.full(o);
     const int iky = ksigned(iy, ny);
     const T ky = T(iky) * dky;
-    const double dt = *rk.dt;
-    cpx<T> s0[EPT], s1[EPT], s2[EPT], sb[EPT];
-    auto ld = [&](int c, int l, int p) {
-      const int line = line0 + l;
-      if (line >= nlines) return zero<T>();
-      return in[c * ifs + (p * nyk + o) * ld1 + line];
-    };
-    // inputs 1-3 are fetched into s1, s2, sb while the transform before
-    // runs (see OpZFwdRK3)
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL, [&](int, int l, int p) { return ld(0, l, p); },
-        [&](int e, int, int, cpx<T> v) { s0[e] = v; },
-        [&](int e, int l, int p) { s1[e] = ld(1, l, p); });
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL, [&](int e, int, int) { return s1[e]; },
-        [&](int e, int, int, cpx<T> v) { s1[e] = v; },
-        [&](int e, int l, int p) { s2[e] = ld(2, l, p); });
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL, [&](int e, int, int) { return s2[e]; },
-        [&](int e, int, int, cpx<T> v) { s2[e] = v; },
-        [&](int e, int l, int p) { sb[e] = ld(3, l, p); });
+    const Lines gi = lines_all((unsigned)ym.nk() * (unsigned)ld1, d.N, nl);
+    const Lines gk = lines_of((unsigned)ny * (unsigned)nkx, zm, false, nl);
+    const cpx<T>* in0 = in + (long long)o * ld1 + line0;
+    const long long base = (long long)iy * nkx + line0;
+    cpx<T> s0[E], s1[E], s2[E], sb[E];
+    auto ld = [&](int c, const Slot& t) { return ln_load<LOGN, T>(gi, in0 + c * ifs, t); };
+    // The v b transforms first: their sum sb is one register array, where
+    // the three tendencies would all be live during them (with the sum last
+    // the pass needs more than 128 registers).  Each input is fetched while
+    // the transform before runs (see OpZFwdRK3).
     // sb = kx G_x + ky G_y + kz G_z  (N_b = -i sb - N^2 v_z)
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL, [&](int e, int, int) { return sb[e]; },
-        [&](int e, int l, int, cpx<T> v) { sb[e] = scale(v, T(line0 + l) * dkx); });
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL, [&](int, int l, int p) { return ld(4, l, p); },
-        [&](int e, int, int, cpx<T> v) { sb[e] = sb[e] + scale(v, ky); });
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL, [&](int, int l, int p) { return ld(5, l, p); },
-        [&](int e, int, int p, cpx<T> v) {
-          sb[e] = sb[e] + scale(v, T(ksigned(p, d.N)) * dkz);
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, d, d.logL, [&](const Slot& t) { return ld(3, t); },
+        [&](const Slot& t, cpx<T> v) { sb[t.e] = scale(v, T(line0 + t.line) * dkx); },
+        [&](const Slot& t) { s0[t.e] = ld(4, t); });
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, d, d.logL, [&](const Slot& t) { return s0[t.e]; },
+        [&](const Slot& t, cpx<T> v) { sb[t.e] = sb[t.e] + scale(v, ky); },
+        [&](const Slot& t) { s1[t.e] = ld(5, t); });
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, d, d.logL, [&](const Slot& t) { return s1[t.e]; },
+        [&](const Slot& t, cpx<T> v) {
+          sb[t.e] = sb[t.e] + scale(v, T(ksigned(t.pos(), d.N)) * dkz);
+        },
+        [&](const Slot& t) { s0[t.e] = ld(0, t); });
+    pin(sb);
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, d, d.logL, [&](const Slot& t) { return s0[t.e]; },
+        [&](const Slot& t, cpx<T> v) { s0[t.e] = v; },
+        [&](const Slot& t) { s1[t.e] = ld(1, t); });
+    pin(s0);
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, d, d.logL, [&](const Slot& t) { return s1[t.e]; },
+        [&](const Slot& t, cpx<T> v) { s1[t.e] = v; },
+        [&](const Slot& t) { s2[t.e] = ld(2, t); });
+    pin(s1);
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, d, d.logL, [&](const Slot& t) { return s2[t.e]; },
+        [&](const Slot& t, cpx<T> v) { s2[t.e] = v; });
+    pin(s2);
+    const RKArgs<T>& rk = late_args<OpZFwdRKStrat>().rk;
+    rk_slots<T, 4, LOGN, LOGE>(
+        d, gk, rk, rk.visc, *rk.dt, mask ? mask + base : nullptr, base, line0, true, iky,
+        [&](const Slot& t, const SlotMode<LOGN, T>& m, cpx<T>* N) {
+          const cpx<T> bs = m.load(rk.src[3]), vzs = m.load(rk.src[2]);
+          N[0] = s0[t.e];
+          N[1] = s1[t.e];
+          N[2] = s2[t.e] + bs;
+          N[3] = scale(mul_i(sb[t.e]), T(-1)) - scale(vzs, N2);
         });
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      int l, p;
-      if (!last_slot<EPT, kT, GEN>(e, d, d.logL, l, p)) continue;
-      const int line = line0 + l;
-      if (line >= nlines || zm.compact(p) < 0) continue;
-      const int idx = (p * ny + iy) * nkx + line;
-      const cpx<T> bs = rk.src[3][idx], vzs = rk.src[2][idx];
-      cpx<T> N[4] = {s0[e], s1[e], s2[e] + bs,
-                     scale(mul_i(sb[e]), T(-1)) - scale(vzs, N2)};
-      if (mask && mask[idx]) N[0] = N[1] = N[2] = N[3] = zero<T>();
-      rk_point<T, 4>(rk, rk.visc, dt, idx, line, iky, ksigned(p, d.N), N);
-    }
   }
 };
 
 // ns2d y-pass, forward, with the Runge-Kutta stage folded in.
 template <typename T>
 struct OpYFwd2RK {
-  static constexpr int kEptDiv = 1;
+  static constexpr bool kMulti = false;
   static constexpr bool kFieldPerBlock = false;
   StridedDesc<T> d;
   const cpx<T>* in;  // W2, 1 field
@@ -793,10 +600,12 @@ struct OpYFwd2RK {
   long long ips = 0, ops = 0;
   const double* bpar = nullptr;
 
-  template <int DIR, int EPT, int kT, bool GEN>
+  template <int DIR, int LOGN, int LOGE>
   __device__ __forceinline__ void run(cpx<T>* buf, const cpx<T>* tw, int o, int line0) const {
-    const int nlines = d.nlines;
-    const cpx<T>* in = this->in + o * ips;
+    constexpr int E = 1 << LOGE;
+    const int nl = d.nlines - line0;
+    const cpx<T>* in0 = in + o * ips + line0;
+    const Lines gi = lines_all(ld2, ny, nl), gk = lines_of(nkx, ym, false, nl);
     double dt;
     Visc visc;
     if (bpar) {
@@ -807,21 +616,14 @@ struct OpYFwd2RK {
       dt = *rk.dt;
       visc = rk.visc;
     }
-    const size_t base = (size_t)o * ops;
-    tile_fft<T, DIR, EPT, kT, GEN>(
-        buf, tw, d, d.logL,
-        [&](int, int l, int p) {
-          const int line = line0 + l;
-          return line < nlines ? in[p * ld2 + line] : zero<T>();
-        },
-        [&](int, int l, int p, cpx<T> v) {
-          const int line = line0 + l;
-          if (line >= nlines || ym.compact(p) < 0) return;
-          const int idx = p * nkx + line;
-          cpx<T> N[1] = {v};
-          if (mask && mask[idx]) N[0] = zero<T>();
-          rk_point<T, 1>(rk, visc, dt, base + idx, line, ksigned(p, ny), 0, N);
-        });
+    cpx<T> s0[E];
+    tile_fft<T, DIR, LOGN, LOGE>(
+        buf, tw, d, d.logL, [&](const Slot& t) { return ln_load<LOGN, T>(gi, in0, t); },
+        [&](const Slot& t, cpx<T> v) { s0[t.e] = v; });
+    pin(s0);
+    rk_slots<T, 1, LOGN, LOGE>(
+        d, gk, rk, visc, dt, mask ? mask + line0 : nullptr, o * ops + line0, line0, false, 0,
+        [&](const Slot& t, const SlotMode<LOGN, T>&, cpx<T>* N) { N[0] = s0[t.e]; });
   }
 };
 

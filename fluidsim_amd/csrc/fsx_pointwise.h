@@ -131,20 +131,70 @@ __device__ __forceinline__ int coarse_index(int ikx, int iky, int ikz, int nkxc,
   return (cz * nyc + cy) * nkxc + ikx;
 }
 
+// A mode by its index in the state arrays.
+template <typename T>
+struct IdxMode {
+  size_t idx;
+  __device__ __forceinline__ cpx<T> load(const cpx<T>* a) const { return a[idx]; }
+  __device__ __forceinline__ void store(cpx<T>* a, cpx<T> v) const { a[idx] = v; }
+};
+
+// State streams a stage reads: S (all but the last RK4 stage) and tmp (RK4
+// after the first stage).  RKStreams holds them, loaded ahead of rk_point by
+// rk_load so that a caller with several modes can have all their loads in
+// flight; RKDirect loads each where it is used (four variables: the streams
+// of one mode alone would push the z-pass beyond its 128 registers).
+template <typename T, int NV>
+struct RKStreams {
+  cpx<T> s[NV], t[NV];
+  template <class Mode>
+  __device__ __forceinline__ cpx<T> S(const RKArgs<T>&, const Mode&, int v) const {
+    return s[v];
+  }
+  template <class Mode>
+  __device__ __forceinline__ cpx<T> tmp(const RKArgs<T>&, const Mode&, int v) const {
+    return t[v];
+  }
+};
+template <typename T>
+struct RKDirect {
+  template <class Mode>
+  __device__ __forceinline__ cpx<T> S(const RKArgs<T>& a, const Mode& m, int v) const {
+    return m.load(a.S[v]);
+  }
+  template <class Mode>
+  __device__ __forceinline__ cpx<T> tmp(const RKArgs<T>& a, const Mode& m, int v) const {
+    return m.load(a.tmp[v]);
+  }
+};
+template <typename T, class Mode>
+__device__ __forceinline__ void rk_load(const RKArgs<T>&, const Mode&, RKDirect<T>&) {}
+template <typename T, int NV, class Mode>
+__device__ __forceinline__ void rk_load(const RKArgs<T>& a, const Mode& m, RKStreams<T, NV>& r) {
+  if (a.stage < 0) return;
+  const bool rk4 = a.scheme == 4;
+  if (!(rk4 && a.stage == 3)) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) r.s[v] = m.load(a.S[v]);
+  }
+  if (rk4 && a.stage > 0) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) r.t[v] = m.load(a.tmp[v]);
+  }
+}
+
 // Integrating-factor Runge-Kutta update of one mode
 // (fluidsim/base/time_stepping/pseudo_spect.py:51-68, 466-517, 898-984):
 // N holds the NV tendencies of the mode (projected here when a.project),
-// E = exp(-dt sigma), E2 = exp(-dt/2 sigma) in FP64.
-// (visc: the viscosities of this mode's run; a.visc except in batches)
-template <typename T, int NV>
+// E = exp(-dt sigma), E2 = exp(-dt/2 sigma) in FP64, only those the stage
+// uses (none in the last RK4 stage); in FP32 E is E2 squared in FP64, far
+// inside the final rounding.  (visc: the viscosities of this mode's run;
+// a.visc except in batches)
+template <typename T, int NV, class Mode, class Streams>
 __device__ __forceinline__ void rk_point(const RKArgs<T>& a, const Visc& visc, double dt,
-                                         size_t idx, int ikx, int iky, int ikz,
-                                         cpx<T>* N) {
+                                         const Mode& m, int ikx, int iky, int ikz,
+                                         const Streams& r, cpx<T>* N) {
   const Box& bx = a.box;
-  const double sig = freq_diss(bx, visc, ikx, iky, ikz);
-  const T e = T(exp(-dt * sig));
-  const T e2 = T(exp(-dt / 2 * sig));
-  const T c6 = T(dt / 6), c3 = T(dt / 3), c2 = T(dt / 2), c1 = T(dt);
   if (a.fc) {
     // tendencies += forcing (ns2d/solver.py:190-191, ns3d/solver.py:243-244)
     const int c = coarse_index(ikx, iky, ikz, a.fnkxc, a.fnyc, a.fnzc);
@@ -155,7 +205,7 @@ __device__ __forceinline__ void rk_point(const RKArgs<T>& a, const Visc& visc, d
   }
 #pragma unroll
   for (int v = 0; v < NV; ++v)
-    if (a.ext[v]) N[v] = N[v] + a.ext[v][idx];
+    if (a.ext[v]) N[v] = N[v] + m.load(a.ext[v]);
   if constexpr (NV >= 3) {
     if (a.project != PROJ_NONE) {
       project3(N[0], N[1], N[2], a.project, ikx, iky, ikz, bx);
@@ -167,55 +217,59 @@ __device__ __forceinline__ void rk_point(const RKArgs<T>& a, const Visc& visc, d
   }
   if (a.stage < 0) {
 #pragma unroll
-    for (int v = 0; v < NV; ++v) a.Nt[v][idx] = N[v];
+    for (int v = 0; v < NV; ++v) m.store(a.Nt[v], N[v]);
     return;
   }
+  const bool rk4 = a.scheme == 4;
+  const bool last = rk4 ? a.stage == 3 : a.stage == 1;
+  T e = T(0), e2 = T(0);
+  if (!(rk4 && last)) {
+    const double sig = freq_diss(bx, visc, ikx, iky, ikz);
+    const double h = exp(-dt / 2 * sig);
+    e2 = T(h);
+    if constexpr (sizeof(T) == 4)
+      e = T(h * h);
+    else if (!rk4 ? last : a.stage != 1)
+      e = T(exp(-dt * sig));
+  }
+  if (!last) {
+    const T c6 = T(dt / 6), c3 = T(dt / 3), c2 = T(dt / 2), c1 = T(dt);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const cpx<T> Nv = N[v], S = r.S(a, m, v);
+      if (!rk4) {
+        m.store(a.t1[v], scale(S + scale(Nv, c2), e2));
+      } else if (a.stage == 0) {
+        m.store(a.tmp[v], scale(S + scale(Nv, c6), e));
+        m.store(a.t1[v], scale(S + scale(Nv, c2), e2));
+      } else {
+        m.store(a.tmp[v], r.tmp(a, m, v) + scale(Nv, c3 * e2));
+        if (a.stage == 1)
+          m.store(a.t1[v], scale(S, e2) + scale(Nv, c2));
+        else
+          m.store(a.t1[v], scale(S, e) + scale(Nv, c1 * e2));
+      }
+    }
+    return;
+  }
+  const T c6 = T(dt / 6), c1 = T(dt);
   cpx<T> Sn[NV];
-  bool last = false;
 #pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const cpx<T> Nv = N[v];
-    if (a.scheme == 4) {
-      if (a.stage == 0) {
-        const cpx<T> S = a.S[v][idx];
-        a.tmp[v][idx] = scale(S + scale(Nv, c6), e);
-        a.t1[v][idx] = scale(S + scale(Nv, c2), e2);
-      } else if (a.stage == 1) {
-        const cpx<T> S = a.S[v][idx];
-        a.tmp[v][idx] = a.tmp[v][idx] + scale(Nv, c3 * e2);
-        a.t1[v][idx] = scale(S, e2) + scale(Nv, c2);
-      } else if (a.stage == 2) {
-        const cpx<T> S = a.S[v][idx];
-        a.tmp[v][idx] = a.tmp[v][idx] + scale(Nv, c3 * e2);
-        a.t1[v][idx] = scale(S, e) + scale(Nv, c1 * e2);
-      } else {
-        Sn[v] = a.tmp[v][idx] + scale(Nv, c6);
-        last = true;
-      }
-    } else {
-      const cpx<T> S = a.S[v][idx];
-      if (a.stage == 0) {
-        a.t1[v][idx] = scale(S + scale(Nv, c2), e2);
-      } else {
-        Sn[v] = scale(S, e) + scale(Nv, c1 * e2);
-        last = true;
+  for (int v = 0; v < NV; ++v)
+    Sn[v] = rk4 ? r.tmp(a, m, v) + scale(N[v], c6)
+                : scale(r.S(a, m, v), e) + scale(N[v], c1 * e2);
+  if constexpr (NV >= 3) {
+    if (a.project != PROJ_NONE) {
+      project3(Sn[0], Sn[1], Sn[2], a.project, ikx, iky, ikz, bx);
+      if (a.no_vz_kz0 && ikz == 0) {
+        Sn[2] = zero<T>();
+        if (NV > 3) Sn[3] = zero<T>();
       }
     }
   }
-  if (last) {
-    if constexpr (NV >= 3) {
-      if (a.project != PROJ_NONE) {
-        project3(Sn[0], Sn[1], Sn[2], a.project, ikx, iky, ikz, bx);
-        if (a.no_vz_kz0 && ikz == 0) {
-          Sn[2] = zero<T>();
-          if (NV > 3) Sn[3] = zero<T>();
-        }
-      }
-    }
 #pragma unroll
-    for (int v = 0; v < NV; ++v) a.S[v][idx] = Sn[v];
-    if (isnan(Sn[0].x) || isnan(Sn[0].y)) atomicOr(a.nanflag, 1u);
-  }
+  for (int v = 0; v < NV; ++v) m.store(a.S[v], Sn[v]);
+  if (isnan(Sn[0].x) || isnan(Sn[0].y)) atomicOr(a.nanflag, 1u);
 }
 
 // One Runge-Kutta stage over the kept modes from a tendency array.
@@ -241,7 +295,9 @@ static __global__ __launch_bounds__(256) void k_rk_stage(RKArgs<T> a) {
       cpx<T> N[NV];
 #pragma unroll
       for (int v = 0; v < NV; ++v) N[v] = a.Nt[v][idx];
-      rk_point<T, NV>(a, a.visc, dt, idx, ikx, iky, ikz, N);
+      const IdxMode<T> m{(size_t)idx};
+      const RKDirect<T> r;
+      rk_point<T, NV>(a, a.visc, dt, m, ikx, iky, ikz, r, N);
     }
   }
 }

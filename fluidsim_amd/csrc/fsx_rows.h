@@ -27,6 +27,7 @@
 #pragma once
 
 #include "fsx_fft.h"
+#include "fsx_tile.h"
 
 namespace fsx {
 
@@ -287,37 +288,6 @@ struct XRNS2D {
     }
   }
 };
-
-// Buffer-resource loads and stores of one complex value.  A raw buffer
-// access whose byte offset is at or beyond the resource's size reads zero
-// and writes nothing, so masked elements (dealiased modes, rows past the
-// end) take the offset kOOB instead of a branch.
-constexpr unsigned kOOB = 0x80000000u;
-typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base,
-                                                          unsigned bytes) {
-  // word 3 = 0x00020000: raw (untyped) 32-bit data format on gfx9 parts
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0,
-                                           (int)bytes, 0x00020000);
-}
-template <typename T>
-__device__ __forceinline__ cpx<T> buf_load(__amdgpu_buffer_rsrc_t r, unsigned off) {
-  if constexpr (sizeof(T) == 4)
-    return __builtin_bit_cast(cpx<T>, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
-  else
-    return __builtin_bit_cast(cpx<T>, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-}
-template <typename T>
-__device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, unsigned off,
-                                          cpx<T> v) {
-  if constexpr (sizeof(T) == 4)
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, v), r, off, 0, 0);
-  else
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), r, off, 0, 0);
-}
-
 
 // Fused row pass, kT threads per workgroup (kT/64 waves, 64/G rows per
 // wave), grid-stride over rows.  LDS: one row buffer per row of a wave.
