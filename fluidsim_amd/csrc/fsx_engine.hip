@@ -134,6 +134,11 @@ int fsx_plan_create(fsx_plan* out, int dim, int nx, int ny, int nz, double Lx,
   hipError_t e = hipSuccess;
   if (p->w1_elems) e = hipMalloc(&p->w1, p->w1_elems * csz);
   if (e == hipSuccess) e = hipMalloc(&p->w2, p->w2_elems * csz);
+  if (e == hipSuccess && dim == 3) {
+    e = hipStreamCreateWithFlags(&p->side, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&p->ev_fork, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&p->ev_join, hipEventDisableTiming);
+  }
   if (e == hipSuccess) e = hipMalloc((void**)&p->d_scal, 32 * sizeof(double));
   if (e == hipSuccess) e = hipMemset(p->d_scal, 0, 32 * sizeof(double));
   if (e != hipSuccess) {
@@ -168,6 +173,9 @@ int fsx_plan_destroy(fsx_plan p) {
   if (p->d_dpart) (void)hipFree(p->d_dpart);
   if (p->d_dout) (void)hipFree(p->d_dout);
   if (p->d_bpar) (void)hipFree(p->d_bpar);
+  if (p->ev_fork) (void)hipEventDestroy(p->ev_fork);
+  if (p->ev_join) (void)hipEventDestroy(p->ev_join);
+  if (p->side) (void)hipStreamDestroy(p->side);
   delete p;
   return 0;
 }

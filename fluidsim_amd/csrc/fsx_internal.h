@@ -126,6 +126,10 @@ struct fsx_plan_s {
   // the inverse and forward y-passes (0: the launcher's choice) and the ns2d
   // inverse with one output field per workgroup
   int ylines_inv, ylines_fwd, ysplit;
+  // second stream of the 3D plane passes (ns3d_planes), forked from and
+  // joined to the caller's stream by events
+  hipStream_t side;
+  hipEvent_t ev_fork, ev_join;
 };
 
 namespace {
@@ -859,6 +863,46 @@ int ns3d_plane_chunk(fsx_plan_s* p, int z0, int nzc, cpx<T>* w2, int nin, int no
   return launch_strided<T, -1>(of, p->ny, nzc, g.mx, nout, p->tw[1], s);
 }
 
+// All planes, in chunks on two streams: even chunks on s, odd ones on the
+// plan's side stream, each stream with its own part of W2.  The y-passes are
+// bound by memory (4.6 TB/s at 512^3 FP32, what a copy of this size reaches),
+// the row pass mostly by its vector instructions (63 % issue), so a row pass
+// that runs beside a y-pass of the other stream hides part of it; and a
+// chunk's W2 (kChunkBytes, two of them at a time) stays in the 256 MB cache
+// between its three passes.  512^3 FP32, three passes of a stage together:
+// 1.99 ms in one go, 1.99 ms in 128 MB chunks on one stream, 1.80 ms in 96 MB
+// chunks on two (2.1 ms in 64 MB chunks: too few workgroups each; 1.99 ms in
+// 128 MB ones: beyond the cache).  Problems whose W2 fits the cache run in
+// one go.
+constexpr double kChunkBytes = 96.0 * (1 << 20);
+
+template <typename T>
+int ns3d_planes(fsx_plan_s* p, int nin, int nout, int want_maxima, hipStream_t s, int strat) {
+  const Geo g = geo<T>(p, true);
+  unsigned long long* mx =
+      want_maxima ? reinterpret_cast<unsigned long long*>(p->d_scal) : nullptr;
+  const long long plane = (long long)nin * p->ny * g.ld2;  // W2 elements
+  const double total = (double)p->nz * plane * sizeof(cpx<T>);
+  int nchunk = (int)std::ceil(total / kChunkBytes);
+  nchunk += nchunk & 1;
+  if (total <= 2 * kChunkBytes || nchunk > p->nz || !p->side)
+    return ns3d_plane_chunk<T>(p, 0, p->nz, W2<T>(p), nin, nout, mx, s, strat);
+  FSX_HIP(hipEventRecord(p->ev_fork, s));
+  FSX_HIP(hipStreamWaitEvent(p->side, p->ev_fork, 0));
+  int rc = 0;
+  const int most = (p->nz + nchunk - 1) / nchunk;  // planes of a chunk
+  for (int i = 0; i < nchunk && !rc; ++i) {
+    const int z0 = (int)((long long)p->nz * i / nchunk);
+    const int z1 = (int)((long long)p->nz * (i + 1) / nchunk);
+    rc = ns3d_plane_chunk<T>(p, z0, z1 - z0, W2<T>(p) + (i & 1) * most * plane, nin, nout, mx,
+                             i & 1 ? p->side : s, strat);
+  }
+  // joined on errors too: the side stream's work precedes what follows on s
+  FSX_HIP(hipEventRecord(p->ev_join, p->side));
+  FSX_HIP(hipStreamWaitEvent(s, p->ev_join, 0));
+  return rc;
+}
+
 // ns3d (strat = 0): z-pass with curl, y-pass, row pass (v x omega, r2c)
 // into W2 fields 0-2.  ns3d.strat (strat = 1): v, omega and b through the
 // z- and y-passes, row pass producing v x omega and v b into W2 fields 0-5.
@@ -889,9 +933,7 @@ int ns3d_front(fsx_plan_s* p, const void* v, int has_f, double fcor,
                    ((nin - 3.0) * g.zm.nk() + (double)nin * p->nz) * sizeof(cpx<T>));
   int rc = launch_strided<T, +1>(op, p->nz, g.ym.nk(), g.mx, nin, p->tw[2], s, true);
   if (rc) return rc;
-  unsigned long long* mx =
-      want_maxima ? reinterpret_cast<unsigned long long*>(p->d_scal) : nullptr;
-  return ns3d_plane_chunk<T>(p, 0, p->nz, W2<T>(p), nin, nout, mx, s, strat);
+  return ns3d_planes<T>(p, nin, nout, want_maxima, s, strat);
 }
 
 template <typename T>

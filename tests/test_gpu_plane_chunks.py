@@ -1,0 +1,96 @@
+"""GPU parity of the 3D plane passes where they run in chunks on two streams
+(W2 larger than two chunks of 96 MB): FP64 tendencies and CFL maxima of ns3d
+and ns3d.strat on a grid of a few unequal chunks against the FP64 oracle
+(relative L2 1e-12, the bar of the other tendency tests), and the fused
+stages captured in a HIP graph against the eager ones, bit for bit, over
+several replays with eager work between them.
+"""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from fluidsim_amd import _lib
+from fluidsim_amd.synthetic import ns3d_spectrum_vv_fft
+from oracle.operators import Oper3D
+from oracle.solvers import NS3D, NS3DStrat
+
+from .gpu_helpers import host, make_plan, rel_l2, to_dev_complex, torch, zeros_complex
+
+pytestmark = pytest.mark.gpu
+
+NX, NY, NZ = 256, 256, 102  # W2 in FP64: 220 MB (ns3d), 257 MB (strat); 25 or 26 planes a chunk
+
+
+def _case(strat):
+    oper = Oper3D(NX, NY, NZ)
+    vv = ns3d_spectrum_vv_fft(NX, NY, NZ, seed=3)
+    if strat:
+        sim = NS3DStrat(oper, N=4.0)
+        sim.init_from_fft(*vv, 0.5 * vv[0])
+    else:
+        sim = NS3D(oper)
+        sim.init_from_vxvyvzfft(*vv)
+    return sim
+
+
+@pytest.mark.parametrize("strat", [False, True])
+def test_chunked_tendency(strat):
+    print(f"case chunked planes strat={strat}", flush=True)
+    sim = _case(strat)
+    ref = sim.tendencies_nonlin(sim.state_spect)
+    plan = make_plan(sim.oper, 8, 7)
+    S = to_dev_complex(sim.state_spect, 8)
+    out = zeros_complex(S.shape, 8)
+    s = _lib.stream_ptr()
+    _lib.call("fsx_reset_maxima", plan.handle, s)
+    if strat:
+        _lib.call("fsx_strat_tendency", plan.handle, _lib.dptr(S), _lib.dptr(out), 0, 0.0, 4.0,
+                  1, 0, 1, s)
+    else:
+        _lib.call("fsx_ns3d_tendency", plan.handle, _lib.dptr(S), _lib.dptr(out), 0, 0.0, 1, s)
+        _lib.call("fsx_project", plan.handle, *(_lib.dptr(out[i]) for i in range(3)), 1, s)
+    assert rel_l2(host(out), ref) < 1e-12
+    sc = (ctypes.c_double * 6)()
+    _lib.call("fsx_get_scalars", plan.handle, sc, s)
+    for i in range(3):
+        v = sim.oper.ifft(sim.state_spect[i])
+        assert sc[i] == pytest.approx(np.abs(v).max(), rel=1e-12)
+
+
+def test_chunked_stages_in_a_graph():
+    t = torch()
+    sim = _case(False)
+    plan = make_plan(sim.oper, 8, 6)
+    S0 = to_dev_complex(sim.state_spect, 8)
+    stream = t.cuda.Stream()
+    sp = _lib.stream_ptr(stream)
+    _lib.call("fsx_set_dt", plan.handle, 1e-3, sp)
+    vc = _lib.doubles([1e-3, 0, 0, 0])
+
+    def buffers():
+        return S0.clone(), t.zeros_like(S0), t.zeros_like(S0)
+
+    def step(S, tmp, t1):
+        for stage in range(4):
+            _lib.call("fsx_ns3d_rk_stage", plan.handle, 4, stage, _lib.dptr(S), _lib.dptr(tmp),
+                      _lib.dptr(t1), 0, 0.0, 1, 0, vc, 0.5, 0.2, sp)
+
+    eager, graph = buffers(), buffers()
+    t.cuda.synchronize()
+    step(*eager)
+    h = ctypes.c_void_p()
+    _lib.call("fsx_graph_begin", sp)
+    try:
+        step(*graph)
+    finally:
+        rc = _lib.get_lib().fsx_graph_end(sp, ctypes.byref(h))
+    _lib.check(rc, "fsx_graph_end")
+    for i in range(3):
+        if i:
+            step(*eager)
+        _lib.call("fsx_graph_launch", h, sp)
+        stream.synchronize()
+        assert t.equal(eager[0], graph[0]), f"replay {i}"
+    _lib.call("fsx_graph_destroy", h)
