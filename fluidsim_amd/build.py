@@ -29,10 +29,6 @@ HIPCC_FLAGS = [
     "--offload-arch=gfx950",
     "-std=c++17",
     "-fPIC",
-    # fuse multiply-adds within expressions only: which ones are fused then
-    # depends on the source and not on what is inlined around it (the tile
-    # settings of the y-passes give the same bits)
-    "-ffp-contract=on",
     # the slot loops around the Runge-Kutta stage index register arrays: they
     # have to be unrolled whatever their size
     "-mllvm", "-pragma-unroll-threshold=65536",

@@ -52,6 +52,12 @@ template <typename T>
 __device__ __forceinline__ cpx<T> scale(cpx<T> a, T s) {
   return mk<T>(a.x * s, a.y * s);
 }
+// scale whose products are not fused into later additions
+template <typename T>
+__device__ __forceinline__ cpx<T> scale_rounded(cpx<T> a, T s) {
+#pragma clang fp contract(off)
+  return mk<T>(a.x * s, a.y * s);
+}
 template <typename T>
 __device__ __forceinline__ cpx<T> conj(cpx<T> a) {
   return mk<T>(a.x, -a.y);
@@ -316,106 +322,317 @@ __device__ __forceinline__ void lds_fft_rows(cpx<T>* buf, int logN, int lines,
 
 // ------------------------------------------------------ mixed-radix lengths
 // Transforms of any length N (grids that are not powers of two) run as
-// Stockham stages of radix 8, 4, 2, 3, 5 and, for any other prime factor p,
-// a direct p-point DFT.  Every stage reads one LDS buffer and writes the
-// other (no register stash across the barrier), with the same index rule as
-// the power-of-two stages: butterfly j (k = j mod Ns) reads positions
-// j + r N/R, applies W_{Ns R}^{r k} and DFT_R, and writes output r to
-// (j - k) R + k + r Ns.  All twiddles are entries of the length-N table
-// tw[m] = exp(-2 pi i m / N).
+// Stockham stages whose radix is one of 2 .. 13, 15 or 16 (products of two
+// coprime factors by the prime-factor index maps, without twiddles; 7, 11 and
+// 13 from the symmetric sums and differences of their inputs) or, for any
+// other prime, a direct DFT, with the same index rule as the power-of-two
+// stages: butterfly j (k = j mod Ns) reads positions j + r N/R, applies
+// W_{Ns R}^{r k} and DFT_R, and writes output r to (j - k) R + k + r Ns.
+// gen_factor picks the fewest stages (240 = 16 15, 192 = 16 12, 160 = 16 10):
+// what a stage costs is its LDS round trip and its barriers.  A thread holds
+// its butterflies (up to kGenRegs values) across the barrier between reading
+// and writing, so a tile that fits the registers needs one LDS buffer; tiles
+// beyond that, and direct stages, read one buffer and write a second.
+//
+// ns3d 240 x 192 x 160 FP64, per stage: rows 1035 -> 270 us, y-inverse 151 ->
+// 160, curl 250 -> 148, z-forward + RK 279 -> 154 us (y-passes and rows of the
+// new figures from 4 overlapping chunks), against radices of at most 8, index
+// divisions per element, full-length transforms of the real rows and loads
+// one at a time.
 constexpr int kMaxStages = 16;
+constexpr int kGenRegs = 16;
 
-// Element (line, pos) of a tile: line-fast (strided passes, `lines` a power
-// of two) or row layout (row passes, row stride ld).
+// Values of a thread's butterflies in a stage of radix r.
+constexpr int gen_held(int r) { return r * (kGenRegs / r); }
+
+// Whether tiles of n elements run in one buffer with kT threads.
+inline bool gen_in_place(const int* rad, int nst, long long n, int kT) {
+  for (int i = 0; i < nst; ++i)
+    if (rad[i] > kGenRegs || n > (long long)kT * gen_held(rad[i])) return false;
+  return true;
+}
+
+// Element (line, pos) of a tile in LDS: line sl + pos sp (strided passes:
+// sl = 1, sp = lines | 1; row passes: sl = row stride, sp = 1).
 struct TileLayout {
-  int logL;  // line-fast: pos << logL | line
-  int ld;    // row layout (logL < 0): line * ld + pos
-  __device__ __forceinline__ int at(int line, int pos) const {
-    return logL >= 0 ? lpad((pos << logL) + line) : line * ld + pos;
-  }
+  int sl, sp;
+  __device__ __forceinline__ int at(int line, int pos) const { return line * sl + pos * sp; }
 };
 
-template <typename T, int DIR, int R>
-__device__ __forceinline__ void gen_butterfly(const cpx<T>* A, cpx<T>* B,
-                                              const TileLayout& lay, const cpx<T>* tw,
-                                              int N, int Ns, int line, int j) {
-  const int NR = N / R;
-  const int k = j % Ns;
-  const int step = NR / Ns;  // N / (Ns R)
-  cpx<T> v[R];
+// n / d for 0 <= n, n d < 2^32, with m = magic_of(d); d = 1 has no magic
+__device__ __forceinline__ unsigned magic_of(unsigned d) { return 0xffffffffu / d + 1u; }
+__device__ __forceinline__ int magic_div(int n, unsigned m, int d) {
+  return d == 1 ? n : (int)__umulhi((unsigned)n, m);
+}
+
+// Index with k mod A = k1 and k mod B = k2 (A, B coprime).
+constexpr int crt_index(int A, int B, int k1, int k2) {
+  for (int k = 0; k < A * B; ++k)
+    if (k % A == k1 && k % B == k2) return k;
+  return 0;
+}
+
+// P-point DFT of an odd prime: with a_m = x_m + x_{P-m}, b_m = x_m - x_{P-m},
+// X_r, X_{P-r} = x_0 + sum_m c_{mr} a_m +- i DIR sum_m s_{mr} b_m.
+template <int P>
+struct PrimeTab;
+template <>
+struct PrimeTab<7> {
+  static constexpr double c[4] = {1, 0.62348980185873353052500488400424, -0.22252093395631440428890256449679,
+                                  -0.90096886790241912623610231950745};
+  static constexpr double s[4] = {0, 0.78183148246802980870844452667406, 0.97492791218182360701813168299393,
+                                  0.43388373911755812047576833284836};
+};
+template <>
+struct PrimeTab<11> {
+  static constexpr double c[6] = {1, 0.84125353283118116886181164891937, 0.41541501300188642552927414922962,
+                                  -0.14231483827328514044379266861637, -0.65486073394528506405692507246629,
+                                  -0.95949297361449738989036805706633};
+  static constexpr double s[6] = {0, 0.54064081745559758210763595431869, 0.90963199535451837141171538307903,
+                                  0.98982144188093273237609203777872, 0.75574957435425828377403584397234,
+                                  0.28173255684142969771141791534662};
+};
+template <>
+struct PrimeTab<13> {
+  static constexpr double c[7] = {1, 0.88545602565320989590037552201510, 0.56806474673115580251180755912752,
+                                  0.12053668025532305334906768745254, -0.35460488704253562596963789260002,
+                                  -0.74851074817110109863463059970135, -0.97094181742605202715698227629379};
+  static constexpr double s[7] = {0, 0.46472317204376854565601533513310, 0.82298386589365639457961742343938,
+                                  0.99270887409805399280075164949252, 0.93501624268541482343978459983783,
+                                  0.66312265824079520237678549266769, 0.23931566428755776714875372626021};
+};
+
+template <typename T, int DIR, int P>
+__device__ __forceinline__ void dft_prime(cpx<T>* v) {
+  constexpr int H = (P - 1) / 2;
+  cpx<T> a[H + 1], b[H + 1];
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    v[r] = A[lay.at(line, j + r * NR)];
-    if (r > 0 && k > 0) {
-      cpx<T> w = tw[r * k * step];
-      if (DIR > 0) w.y = -w.y;
-      v[r] = v[r] * w;
-    }
+  for (int m = 1; m <= H; ++m) {
+    a[m] = v[m] + v[P - m];
+    b[m] = v[m] - v[P - m];
   }
+  const cpx<T> x0 = v[0];
+#pragma unroll
+  for (int m = 1; m <= H; ++m) v[0] = v[0] + a[m];
+#pragma unroll
+  for (int r = 1; r <= H; ++r) {
+    cpx<T> t = x0, u = zero<T>();
+#pragma unroll
+    for (int m = 1; m <= H; ++m) {
+      const int q = (m * r) % P, qs = q <= H ? q : P - q;
+      const T c = T(PrimeTab<P>::c[qs]), s = T(q <= H ? PrimeTab<P>::s[qs] : -PrimeTab<P>::s[qs]);
+      t = mk<T>(fma_t(c, a[m].x, t.x), fma_t(c, a[m].y, t.y));
+      u = mk<T>(fma_t(s, b[m].x, u.x), fma_t(s, b[m].y, u.y));
+    }
+    u = rot90<T, DIR>(u);
+    v[r] = t + u;
+    v[P - r] = t - u;
+  }
+}
+
+// 9-point DFT as 3 x 3 (n = 3 n1 + n2, k = k1 + 3 k2) with W9^{n2 k1} between.
+template <typename T, int DIR>
+__device__ __forceinline__ void dft9(cpx<T>* v) {
+  constexpr T c1 = T(0.76604444311897803520239265055542), s1 = T(0.64278760968653932632264340990726);
+  constexpr T c2 = T(0.17364817766693034885171662676931), s2 = T(0.98480775301220805936674302458952);
+  constexpr T c4 = T(-0.93969262078590838405410927732473), s4 = T(0.34202014332566873304409961468226);
+  cpx<T> y[3][3];
+#pragma unroll
+  for (int n2 = 0; n2 < 3; ++n2) {
+#pragma unroll
+    for (int n1 = 0; n1 < 3; ++n1) y[n2][n1] = v[3 * n1 + n2];
+    dft3<T, DIR>(y[n2]);
+  }
+  auto tw = [](cpx<T> x, T c, T s) {
+    const T w = DIR < 0 ? -s : s;
+    return mk<T>(fma_t(x.x, c, -(x.y * w)), fma_t(x.x, w, x.y * c));
+  };
+  y[1][1] = tw(y[1][1], c1, s1);
+  y[1][2] = tw(y[1][2], c2, s2);
+  y[2][1] = tw(y[2][1], c2, s2);
+  y[2][2] = tw(y[2][2], c4, s4);
+#pragma unroll
+  for (int k1 = 0; k1 < 3; ++k1) {
+    cpx<T> b[3] = {y[0][k1], y[1][k1], y[2][k1]};
+    dft3<T, DIR>(b);
+#pragma unroll
+    for (int k2 = 0; k2 < 3; ++k2) v[k1 + 3 * k2] = b[k2];
+  }
+}
+
+template <typename T, int DIR, int R>
+__device__ __forceinline__ void dft_any(cpx<T>* v);
+
+// A B-point DFT of coprime A, B (prime-factor maps): n = B n1 + A n2, output
+// k = k1 mod A = k2 mod B; no twiddles between the two.
+template <typename T, int DIR, int A, int B>
+__device__ __forceinline__ void dft_pf(cpx<T>* v) {
+  cpx<T> y[A][B];
+#pragma unroll
+  for (int n2 = 0; n2 < B; ++n2) {
+    cpx<T> a[A];
+#pragma unroll
+    for (int n1 = 0; n1 < A; ++n1) a[n1] = v[(B * n1 + A * n2) % (A * B)];
+    dft_any<T, DIR, A>(a);
+#pragma unroll
+    for (int k1 = 0; k1 < A; ++k1) y[k1][n2] = a[k1];
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < A; ++k1) {
+    dft_any<T, DIR, B>(y[k1]);
+#pragma unroll
+    for (int k2 = 0; k2 < B; ++k2) v[crt_index(A, B, k1, k2)] = y[k1][k2];
+  }
+}
+
+template <typename T, int DIR, int R>
+__device__ __forceinline__ void dft_any(cpx<T>* v) {
   if constexpr (R == 3)
     dft3<T, DIR>(v);
   else if constexpr (R == 5)
     dft5<T, DIR>(v);
+  else if constexpr (R == 6)
+    dft_pf<T, DIR, 2, 3>(v);
+  else if constexpr (R == 7 || R == 11 || R == 13)
+    dft_prime<T, DIR, R>(v);
+  else if constexpr (R == 9)
+    dft9<T, DIR>(v);
+  else if constexpr (R == 10)
+    dft_pf<T, DIR, 2, 5>(v);
+  else if constexpr (R == 12)
+    dft_pf<T, DIR, 4, 3>(v);
+  else if constexpr (R == 15)
+    dft_pf<T, DIR, 3, 5>(v);
   else
     dftR<T, DIR, R>(v);
-  const int o = (j - k) * R + k;
+}
+
+// One stage of radix R over `lines` lines: A -> B (the same buffer where the
+// butterflies of all threads fit their registers).  The twiddles are entries
+// of tw[m] = exp(-2 pi i m / (N tws)).
+struct GenStage {
+  int N, Ns, lines, logL;  // logL >= 0: line-fast thread map, lines = 2^logL
+  int tws;
+};
+template <typename T, int DIR, int R, int kT>
+__device__ __forceinline__ void gen_stage(const cpx<T>* A, cpx<T>* B, const TileLayout& lay,
+                                          const cpx<T>* tw, const GenStage& g) {
+  constexpr int NB = kGenRegs / R;
+  const int NR = g.N / R, Ns = g.Ns;
+  const int nb = NR * g.lines, step = NR / Ns * g.tws;
+  const unsigned mNs = magic_of(Ns), mNR = magic_of(NR);
+  // (one turn where A is B)
+  for (int b0 = threadIdx.x; b0 < nb + (int)threadIdx.x; b0 += NB * kT) {
+    cpx<T> v[NB][R];
+    int o[NB], ks[NB];
 #pragma unroll
-  for (int r = 0; r < R; ++r) B[lay.at(line, o + r * Ns)] = v[r];
+    for (int i = 0; i < NB; ++i) {
+      const int b = b0 + i * kT;
+      if (i > 0 && b >= nb) break;
+      int line, j;
+      if (g.logL >= 0) {
+        line = b & (g.lines - 1);
+        j = b >> g.logL;
+      } else {
+        line = magic_div(b, mNR, NR);
+        j = b - line * NR;
+      }
+      const int k = j - magic_div(j, mNs, Ns) * Ns;
+      ks[i] = k * step;
+      o[i] = lay.at(line, (j - k) * R + k);
+      if (b < nb) {
+        const cpx<T>* a = A + lay.at(line, j);
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[i][r] = a[r * NR * lay.sp];
+        if (Ns > 1) {
+#pragma unroll
+          for (int r = 1; r < R; ++r) {
+            cpx<T> w = tw[r * ks[i]];
+            if (DIR > 0) w.y = -w.y;
+            v[i][r] = v[i][r] * w;
+          }
+        }
+        dft_any<T, DIR, R>(v[i]);
+      }
+    }
+    if (A == B) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int b = b0 + i * kT;
+      if (b < nb) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) B[o[i] + r * Ns * lay.sp] = v[i][r];
+      }
+    }
+  }
 }
 
 // Direct DFT of a prime radix R without a dedicated butterfly: output r of
 // butterfly j is sum_m (x_m W_{Ns R}^{m k}) W_R^{m r}.
-template <typename T, int DIR>
+template <typename T, int DIR, int kT>
 __device__ __forceinline__ void gen_direct(const cpx<T>* A, cpx<T>* B, const TileLayout& lay,
-                                           const cpx<T>* tw, int N, int R, int Ns,
-                                           int line, int j) {
-  const int NR = N / R;
-  const int k = j % Ns;
-  const int step = NR / Ns;
-  const int o = (j - k) * R + k;
-  for (int r = 0; r < R; ++r) {
-    cpx<T> acc = zero<T>();
-    for (int m = 0; m < R; ++m) {
-      cpx<T> x = A[lay.at(line, j + m * NR)];
-      cpx<T> w = tw[m * k * step];
-      cpx<T> u = tw[((m * r) % R) * NR];
-      if (DIR > 0) {
-        w.y = -w.y;
-        u.y = -u.y;
+                                           const cpx<T>* tw, const GenStage& g, int R) {
+  const int NR = g.N / R, Ns = g.Ns;
+  const int nb = NR * g.lines, step = NR / Ns;
+  for (int b = threadIdx.x; b < nb; b += kT) {
+    const int line = g.logL >= 0 ? b & (g.lines - 1) : b / NR;
+    const int j = g.logL >= 0 ? b >> g.logL : b - line * NR;
+    const int k = j % Ns;
+    const int o = (j - k) * R + k;
+    for (int r = 0; r < R; ++r) {
+      cpx<T> acc = zero<T>();
+      int q = 0;  // m r mod R
+      for (int m = 0; m < R; ++m) {
+        cpx<T> w = tw[m * k * step * g.tws];
+        cpx<T> u = tw[q * NR * g.tws];
+        if (DIR > 0) {
+          w.y = -w.y;
+          u.y = -u.y;
+        }
+        acc = acc + (A[lay.at(line, j + m * NR)] * w) * u;
+        q += r;
+        if (q >= R) q -= R;
       }
-      acc = acc + (x * w) * u;
+      B[lay.at(line, o + r * Ns)] = acc;
     }
-    B[lay.at(line, o + r * Ns)] = acc;
   }
 }
 
-// All stages of `lines` transforms of length N over the tile in A (B is the
-// second buffer).  The caller synchronises before; returns the buffer that
-// holds the result, after a barrier.
+// All stages of `lines` transforms of length N over the tile in A (B: the
+// second buffer, or A), kT threads.  The caller synchronises before; returns the
+// buffer that holds the result, after a barrier.
 template <typename T, int DIR, int kT>
-__device__ cpx<T>* gen_fft(cpx<T>* A, cpx<T>* B, const TileLayout& lay, const cpx<T>* tw,
-                           int N, int lines, int nst, const int* rad) {
+__device__ __forceinline__ cpx<T>* gen_fft(cpx<T>* A, cpx<T>* B, const TileLayout& layout,
+                                           const cpx<T>* tw, int tws, int N, int lines, int logL,
+                                           int nst, const int* rad) {
   int Ns = 1;
   for (int s = 0; s < nst; ++s) {
     const int R = rad[s];
-    const int nb = (N / R) * lines;
-    for (int b = threadIdx.x; b < nb; b += kT) {
-      int line, j;
-      if (lay.logL >= 0) {
-        line = b & ((1 << lay.logL) - 1);
-        j = b >> lay.logL;
-      } else {
-        line = b / (N / R);
-        j = b - line * (N / R);
-      }
-      switch (R) {
-        case 2: gen_butterfly<T, DIR, 2>(A, B, lay, tw, N, Ns, line, j); break;
-        case 3: gen_butterfly<T, DIR, 3>(A, B, lay, tw, N, Ns, line, j); break;
-        case 4: gen_butterfly<T, DIR, 4>(A, B, lay, tw, N, Ns, line, j); break;
-        case 5: gen_butterfly<T, DIR, 5>(A, B, lay, tw, N, Ns, line, j); break;
-        case 8: gen_butterfly<T, DIR, 8>(A, B, lay, tw, N, Ns, line, j); break;
-        default: gen_direct<T, DIR>(A, B, lay, tw, N, R, Ns, line, j); break;
-      }
+    // opaque to the optimizer: the strides of every radix below would
+    // otherwise be computed ahead of the loop and kept in registers
+    int n = __builtin_amdgcn_readfirstlane(N), sp = __builtin_amdgcn_readfirstlane(layout.sp);
+    asm volatile("" : "+s"(n), "+s"(sp));
+    const TileLayout lay{layout.sl, __builtin_amdgcn_readfirstlane(sp)};
+    const GenStage g{__builtin_amdgcn_readfirstlane(n), Ns, lines, logL, tws};
+    switch (R) {
+#define FSX_GEN_RADIX(r) \
+  case r: gen_stage<T, DIR, r, kT>(A, B, lay, tw, g); break;
+      FSX_GEN_RADIX(2)
+      FSX_GEN_RADIX(3)
+      FSX_GEN_RADIX(4)
+      FSX_GEN_RADIX(5)
+      FSX_GEN_RADIX(6)
+      FSX_GEN_RADIX(7)
+      FSX_GEN_RADIX(8)
+      FSX_GEN_RADIX(9)
+      FSX_GEN_RADIX(10)
+      FSX_GEN_RADIX(11)
+      FSX_GEN_RADIX(12)
+      FSX_GEN_RADIX(13)
+      FSX_GEN_RADIX(15)
+      FSX_GEN_RADIX(16)
+#undef FSX_GEN_RADIX
+      default: gen_direct<T, DIR, kT>(A, B, lay, tw, g, R); break;
     }
     __syncthreads();
     cpx<T>* t = A;
@@ -426,37 +643,48 @@ __device__ cpx<T>* gen_fft(cpx<T>* A, cpx<T>* B, const TileLayout& lay, const cp
   return A;
 }
 
-// Stage radices of a length-n transform (host): 8s, then 4 or 2, then 3s,
-// 5s and the remaining primes in increasing order.  Returns the number of
-// stages, or -1 when more than kMaxStages would be needed.
+// Stage radices of a length-n transform (host): the fewest stages of the
+// butterflies above, the most even of those (smallest sum of radices), larger
+// radices first; other primes are stages of their own.  Returns the number
+// of stages, or -1 when more than kMaxStages would be needed.
+inline void gen_split(int n, int maxr, int* cur, int nc, int sum, int* best, int& nbest,
+                      int& sbest) {
+  if (n == 1) {
+    if (nc < nbest || (nc == nbest && sum < sbest)) {
+      nbest = nc;
+      sbest = sum;
+      for (int i = 0; i < nc; ++i) best[i] = cur[i];
+    }
+    return;
+  }
+  if (nc >= nbest) return;
+  for (int r = maxr; r >= 2; --r) {
+    if (r == 14 || n % r != 0) continue;
+    cur[nc] = r;
+    gen_split(n / r, r, cur, nc + 1, sum + r, best, nbest, sbest);
+  }
+}
 inline int gen_factor(int n, int* rad) {
+  // primes without a butterfly
+  int big[kMaxStages], nbig = 0, m = n;
+  for (int p : {2, 3, 5, 7, 11, 13})
+    while (m % p == 0) m /= p;
+  int smooth = n / m;
+  for (int p = 17; m > 1; p += 2) {
+    if ((long long)p * p > m) p = m;
+    while (m % p == 0) {
+      if (nbig >= kMaxStages) return -1;
+      big[nbig++] = p;
+      m /= p;
+    }
+  }
+  int cur[kMaxStages + 1], best[kMaxStages + 1];
+  int nbest = kMaxStages + 1, sbest = 0;
+  gen_split(smooth, 16, cur, 0, 0, best, nbest, sbest);
+  if (nbest + nbig > kMaxStages) return -1;
   int ns = 0;
-  int p2 = 0;
-  while (n % 2 == 0) {
-    n /= 2;
-    ++p2;
-  }
-  while (p2 >= 3) {
-    if (ns >= kMaxStages) return -1;
-    rad[ns++] = 8;
-    p2 -= 3;
-  }
-  if (p2 > 0) {
-    if (ns >= kMaxStages) return -1;
-    rad[ns++] = 1 << p2;
-  }
-  for (int p = 3; n > 1; p += 2) {
-    while (n % p == 0) {
-      if (ns >= kMaxStages) return -1;
-      rad[ns++] = p;
-      n /= p;
-    }
-    if ((long long)p * p > n && n > 1) {
-      if (ns >= kMaxStages) return -1;
-      rad[ns++] = n;
-      n = 1;
-    }
-  }
+  for (int i = 0; i < nbest; ++i) rad[ns++] = best[i];
+  for (int i = 0; i < nbig; ++i) rad[ns++] = big[i];
   return ns;
 }
 

@@ -282,10 +282,10 @@ int launch_strided(Op& op, int N, int nouter, int nlines, int nf, const void* tw
     L = tile / N;
     op.d.nst = 0;
   } else {
-    // mixed-radix stages in LDS: tiles of half the size (two buffers)
+    // mixed-radix stages in LDS: as many elements as the slots hold
     op.d.nst = gen_factor(N, op.d.rad);
     if (op.d.nst < 0) return fail(FSX_ERR_ARG, "transform length has too many factors");
-    L = (kGenThr << LOGE) / 2 / N;
+    L = (kGenThr << LOGE) / N;
     if (L < 1) return fail(FSX_ERR_ARG, "transform length exceeds the tile");
   }
   while (L & (L - 1)) L &= L - 1;  // power of two
@@ -336,8 +336,10 @@ int launch_strided(Op& op, int N, int nouter, int nlines, int nf, const void* tw
                      (p2 ? (size_t)strided_tile<T>() : (size_t)kGenThr << LOGE);
     if (op.d.stack) need *= line_mul<Op>::value;
   }
+
   if (!p2) {
-    const size_t lds = (2 * (need + need / 32 + 1) + N) * sizeof(cpx<T>);
+    op.d.inplace = gen_in_place(op.d.rad, op.d.nst, (long long)need, kGenThr);
+    const size_t lds = ((op.d.inplace ? 1 : 2) * N * ((need / N) | 1) + N) * sizeof(cpx<T>);
     return launch_strided_kernel<T, DIR, 0, LOGE>(op, kGenThr, lds, blocks, nfb, s);
   }
   switch (logN) {
@@ -362,17 +364,25 @@ template <typename T, class Op>
 int launch_xpass_gen(Op& op, int nx, int nrows, int nf_in, int nf_out, int mx_in,
                      int ld_in, int mx_out, int ld_out, long long ifs, long long ofs,
                      T scl, const void* tw, hipStream_t s) {
-  // two buffers of complex rows in the workgroup's LDS, after the twiddles
-  const int tile = (int)((kLdsMax / sizeof(cpx<T>) - (size_t)nx) / 2);
   const int nfm = nf_in > nf_out ? nf_in : nf_out;
-  const int ld = nx + 1;
-  if (nfm * ld > tile) return fail(FSX_ERR_ARG, "row pass exceeds the tile");
-  int RB = tile / (nfm * ld);
+  // rows of up to this length are taken
+  const int tile = (int)((kLdsMax / sizeof(cpx<T>) - (size_t)nx) / 2);
+  if (nfm * (nx + 1) > tile) return fail(FSX_ERR_ARG, "row pass exceeds the tile");
+  const int M = nx % 2 == 0 ? nx / 2 : nx;
+  op.d.nst = gen_factor(M, op.d.rad);
+  if (op.d.nst < 0) return fail(FSX_ERR_ARG, "row length has too many factors");
+  // rows per workgroup: as many as the threads' registers hold (one LDS
+  // buffer, at most 48 KB so that three workgroups share a CU), else one row
+  const int most = 48 * 1024 / (int)sizeof(cpx<T>);
+  int RB = most / (nfm * M);
+  while (RB > 1 && !gen_in_place(op.d.rad, op.d.nst, (long long)nfm * RB * M, kGenThr)) --RB;
+  if (RB < 1) RB = 1;
   if (RB > nrows) RB = nrows > 0 ? nrows : 1;
   while (RB > 1 && (nrows + RB - 1) / RB < kMinBlocks) RB = (RB + 1) / 2;
+  op.d.inplace = gen_in_place(op.d.rad, op.d.nst, (long long)nfm * RB * M, kGenThr);
   op.d.nx = nx;
   op.d.lognx = -1;
-  op.d.M = 0;
+  op.d.M = M;
   op.d.logM = -1;
   op.d.RB = RB;
   op.d.logRB = -1;
@@ -387,12 +397,10 @@ int launch_xpass_gen(Op& op, int nx, int nrows, int nf_in, int nf_out, int mx_in
   op.d.ofs = ofs;
   op.d.scale = scl;
   op.d.tw = reinterpret_cast<const cpx<T>*>(tw);
-  op.d.nst = gen_factor(nx, op.d.rad);
-  if (op.d.nst < 0) return fail(FSX_ERR_ARG, "row length has too many factors");
   if (nrows <= 0) return 0;
   const long long blocks = (nrows + RB - 1) / RB;
-  const size_t lds = ((size_t)2 * nfm * RB * ld + nx) * sizeof(cpx<T>);
-  auto kern = k_xpass_gen<T, kXThr, Op>;
+  const size_t lds = ((size_t)(op.d.inplace ? 1 : 2) * nfm * RB * M + nx) * sizeof(cpx<T>);
+  auto kern = k_xpass_gen<T, Op>;
   static size_t lds_set = 0;
   if (lds > kLdsMax) return fail(FSX_ERR_ARG, "pass needs more LDS than a workgroup has");
   if (lds > lds_set) {
@@ -402,7 +410,7 @@ int launch_xpass_gen(Op& op, int nx, int nrows, int nf_in, int nf_out, int mx_in
   }
   int rc = tm_pre(s);
   if (rc) return rc;
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kXThr), lds, s, op);
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kGenThr), lds, s, op);
   FSX_HIP(hipGetLastError());
   return tm_post(s);
 }

@@ -45,7 +45,10 @@ __device__ __forceinline__ int xcd_remap(int b, int nb) {
 // Strided pass.  LOGN > 0: length 2^LOGN, N L / 2^LOGE threads (4 L where
 // the op stacks its outputs); LOGN = 0: any length, kGenThr threads.
 template <typename T, int DIR, int LOGN, int LOGE, class Op>
-static __global__ __launch_bounds__((LOGN > 0 ? strided_tile<T, LOGN, Op>() >> LOGE : kGenThr))
+// (mixed radix: at least 4, FP64 3, or 2 where transforms are kept, waves per SIMD; the
+// widest of the many butterflies would take 200 to 500 registers otherwise)
+static __global__ __launch_bounds__((LOGN > 0 ? strided_tile<T, LOGN, Op>() >> LOGE : kGenThr),
+                                    (LOGN > 0 ? 1 : (Op::kMulti ? 2 : (sizeof(T) == 8 ? 3 : 4))))
 void k_strided(Op op) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const StridedDesc<T>& d = op.d;
@@ -231,7 +234,12 @@ struct OpZInvCurl {
     cpx<T> sVz[E], sv[E], sVy[E];
     auto ld = [&](int c, const Slot& t) { return ln_load<LOGN, T>(gi, in0 + c * ifs, t); };
     auto st = [&](int c, const Slot& t, cpx<T> v) { ln_store<LOGN, T>(go, out0 + c * ofs, t, v); };
-    auto kz_of = [&](const Slot& t) { return T(ksigned(t.pos(), nz)) * dkz; };
+    // (not shared between its two uses: eight registers for a transform)
+    auto kz_of = [&](const Slot& t) {
+      int p = t.pos();
+      asm volatile("" : "+v"(p));
+      return T(ksigned(p, nz)) * dkz;
+    };
     auto kx_of = [&](const Slot& t) { return T(line0 + t.line) * dkx; };
     // Each input is loaded once, into sv (vy, then vx) or sVz (b, once Vz
     // is no longer needed), while the transform before the one that first
@@ -303,7 +311,8 @@ struct OpYInv2NS {
   AxisMap ym;
   T dkx, dky;
 
-  // multiplier (without i) of output c at (line, p)
+  // multiplier (without i) of output c at (line, p); applied with
+  // scale_rounded, so that the forms of the pass below give the same bits
   __device__ __forceinline__ T factor(int c, int line, int p) const {
     const T kx = T(line) * dkx, ky = T(ksigned(p, ny)) * dky;
     if (c >= 2) return c == 2 ? kx : ky;
@@ -328,7 +337,7 @@ struct OpYInv2NS {
           [&](const Slot& t) {
             const Slot u{t.e, t.line & lm, t.j, t.pr};
             const cpx<T> r = ln_load<LOGN, T>(gi, in0, u);
-            return mul_i(scale(r, factor(t.line >> d.logL, line0 + u.line, t.pos())));
+            return mul_i(scale_rounded(r, factor(t.line >> d.logL, line0 + u.line, t.pos())));
           },
           [&](const Slot& t, cpx<T> v) {
             const Slot u{t.e, t.line & lm, t.j, t.pr};
@@ -351,7 +360,7 @@ struct OpYInv2NS {
         buf, tw, d, d.logL,
         [&](const Slot& t) {
           sr[t.e] = ln_load<LOGN, T>(gi, in0, t);
-          return mul_i(scale(sr[t.e], factor(0, line0 + t.line, t.pos())));
+          return mul_i(scale_rounded(sr[t.e], factor(0, line0 + t.line, t.pos())));
         },
         [&](const Slot& t, cpx<T> v) { ln_store<LOGN, T>(go, out0, t, v); });
 #pragma unroll
@@ -359,7 +368,7 @@ struct OpYInv2NS {
       tile_fft<T, DIR, LOGN, LOGE>(
           buf, tw, d, d.logL,
           [&](const Slot& t) {
-            return mul_i(scale(sr[t.e], factor(c, line0 + t.line, t.pos())));
+            return mul_i(scale_rounded(sr[t.e], factor(c, line0 + t.line, t.pos())));
           },
           [&](const Slot& t, cpx<T> v) { ln_store<LOGN, T>(go, out0 + c * ofs, t, v); });
   }
@@ -386,7 +395,7 @@ struct OpYInv2NSOne : OpYInv2NS<T> {
         buf, tw, d, d.logL,
         [&](const Slot& t) {
           const cpx<T> r = ln_load<LOGN, T>(gi, in0, t);
-          return mul_i(scale(r, this->factor(c, line0 + t.line, t.pos())));
+          return mul_i(scale_rounded(r, this->factor(c, line0 + t.line, t.pos())));
         },
         [&](const Slot& t, cpx<T> v) { ln_store<LOGN, T>(go, out0, t, v); });
   }
@@ -640,7 +649,7 @@ struct XDesc {
   T scale;             // applied to the r2c output
   const cpx<T>* tw;    // exp(-2 pi i m / nx), m < nx (copied to LDS)
   // mixed-radix stages of a length-nx complex transform (k_xpass_gen)
-  int nst;
+  int nst, inplace;
   int rad[kMaxStages];
 };
 
@@ -807,79 +816,138 @@ void k_xpass(Op op) {
   }
 }
 
-// Row pass of any length nx (grids that are not powers of two): each real
-// row is one length-nx complex transform in LDS (gen_fft, row layout with
-// stride nx + 1).  The c2r input is the half spectrum extended by Hermitian
-// symmetry, X[nx - k] = conj X[k]; the real part of the inverse transform is
-// the row (the imaginary parts of X[0] and, for even nx, X[nx/2] drop out,
-// as in numpy's irfft).  The products run per point (Op::point) on the real
-// parts; the forward transform of the real product rows keeps kx < mx_out.
-// Rows per workgroup: d.RB (any count), fields stacked as rows f RB + r.
-template <typename T, int kT, class Op>
-static __global__ __launch_bounds__(kT) void k_xpass_gen(Op op) {
+// Row pass of any length nx (grids that are not powers of two).  Even nx:
+// a real row is one complex transform of length M = nx/2, z[j] = x[2j] +
+// i x[2j+1], with the pairing of k and M - k before and after it as in
+// k_xpass (computed per element, both operands read from memory, the second
+// from cache).  Odd nx: one complex transform of length M = nx of the half
+// spectrum extended by Hermitian symmetry, whose real part is the row (the
+// imaginary part of X[0] drops out, as in numpy's irfft).  The products run
+// per point (Op::point).  Rows per workgroup: d.RB (any count), fields
+// stacked as rows f RB + r of stride M in one or two LDS buffers (gen_fft).
+template <typename T, class Op>
+static __global__ __launch_bounds__(kGenThr, 4) void k_xpass_gen(Op op) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
+  constexpr int kT = kGenThr;
   const XDesc<T>& d = op.d;
-  const int nx = d.nx, ld = nx + 1, RB = d.RB;
+  const int nx = d.nx, RB = d.RB, M = d.M;
+  const bool half = M != nx;
   cpx<T>* s_tw = reinterpret_cast<cpx<T>*>(smem_raw);
   const int nfm = d.nf_in > d.nf_out ? d.nf_in : d.nf_out;
   cpx<T>* A = s_tw + nx;
-  cpx<T>* B = A + nfm * RB * ld;
+  cpx<T>* B = d.inplace ? A : A + nfm * RB * M;
   const int row0 = blockIdx.x * RB;
   const int tid = threadIdx.x;
-  const TileLayout lay{-1, ld};
+  const TileLayout lay{M, 1};
+  const unsigned mM = magic_of(M), mRB = magic_of(RB);
   for (int i = tid; i < nx; i += kT) s_tw[i] = d.tw[i];
-  const int n_in = d.nf_in * RB * nx;
-  for (int idx = tid; idx < n_in; idx += kT) {
-    const int lr = idx / nx, x = idx - lr * nx;
-    const int f = lr / RB, row = row0 + (lr - f * RB);
-    cpx<T> v = zero<T>();
-    if (row < d.nrows) {
+  __syncthreads();
+  const int n_in = d.nf_in * RB * M;
+  // the loads of kU elements of a thread are issued before any is used; what
+  // is masked (dealiased modes, rows past the end) reads element 0 instead
+  constexpr int kU = 4;
+  for (int base = tid; base < n_in; base += kU * kT) {
+    cpx<T> Xk[kU], Xm[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int idx = base + u * kT < n_in ? base + u * kT : 0;
+      const int lr = magic_div(idx, mM, M), x = idx - lr * M;
+      const int f = magic_div(lr, mRB, RB), row = row0 + (lr - f * RB);
+      const bool in = row < d.nrows;
       if constexpr (Op::kInv) {
-        const int k = x <= nx / 2 ? x : nx - x;
-        if (k < d.mx_in) v = op.in[f * d.ifs + (long long)row * d.ld_in + k];
-        if (x > nx / 2) v = conj(v);
+        const cpx<T>* src = op.in + (in ? f * d.ifs + (long long)row * d.ld_in : 0);
+        const int k = half || x <= nx / 2 ? x : nx - x;
+        const bool okk = in && k < d.mx_in, okm = in && half && M - x < d.mx_in;
+        Xk[u] = src[okk ? k : 0];
+        Xm[u] = src[okm ? M - x : 0];
+        if (!okk) Xk[u] = zero<T>();
+        if (!okm) Xm[u] = zero<T>();
       } else {
-        v.x = op.inr[f * d.ifs + (long long)row * nx + x];
+        const T* src = op.inr + (in ? f * d.ifs + (long long)row * nx : 0);
+        Xk[u] = half ? mk<T>(src[2 * x], src[2 * x + 1]) : mk<T>(src[x], T(0));
+        if (!in) Xk[u] = zero<T>();
       }
     }
-    A[lr * ld + x] = v;
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int idx = base + u * kT;
+      if (idx >= n_in) break;
+      const int x = idx - magic_div(idx, mM, M) * M;
+      cpx<T> v = Xk[u];
+      if constexpr (Op::kInv) {
+        if (half) {
+          if (x == 0) Xk[u].y = Xm[u].y = T(0);
+          const cpx<T> w = s_tw[x];
+          const cpx<T> dk = Xk[u] - conj(Xm[u]);
+          v = (Xk[u] + conj(Xm[u])) + mul_i(conj(w) * dk);
+        } else if (x > nx / 2) {
+          v = conj(v);
+        }
+      }
+      A[idx] = v;
+    }
   }
   __syncthreads();
   cpx<T>* res = A;
   if constexpr (Op::kInv) {
-    res = gen_fft<T, +1, kT>(A, B, lay, s_tw, nx, d.nf_in * RB, d.nst, d.rad);
+    res = gen_fft<T, +1, kT>(A, B, lay, s_tw, half ? 2 : 1, M, d.nf_in * RB, -1, d.nst, d.rad);
     if constexpr (Op::kStoreReal) {
       for (int idx = tid; idx < n_in; idx += kT) {
-        const int lr = idx / nx, x = idx - lr * nx;
-        const int f = lr / RB, row = row0 + (lr - f * RB);
-        if (row < d.nrows) op.outr[f * d.ofs + (long long)row * nx + x] = res[lr * ld + x].x;
+        const int lr = magic_div(idx, mM, M), x = idx - lr * M;
+        const int f = magic_div(lr, mRB, RB), row = row0 + (lr - f * RB);
+        if (row >= d.nrows) continue;
+        T* dst = op.outr + f * d.ofs + (long long)row * nx;
+        const cpx<T> v = res[idx];
+        if (half) {
+          dst[2 * x] = v.x;
+          dst[2 * x + 1] = v.y;
+        } else {
+          dst[x] = v.x;
+        }
       }
       return;
     } else {
       T m[3] = {0, 0, 0};
-      for (int idx = tid; idx < RB * nx; idx += kT) {
-        const int r = idx / nx, x = idx - r * nx;
-        T v[8];
-        for (int c = 0; c < d.nf_in && c < 8; ++c) v[c] = res[(c * RB + r) * ld + x].x;
+      const int fs = RB * M;  // elements per field
+      for (int idx = tid; idx < fs; idx += kT) {
+        const int r = magic_div(idx, mM, M);
+        T v[8], u[8];
+        for (int c = 0; c < d.nf_in && c < 8; ++c) {
+          const cpx<T> z = res[c * fs + idx];
+          v[c] = z.x;
+          u[c] = z.y;
+        }
         T mm[3] = {0, 0, 0};
         op.point(v, mm);
+        if (half) op.point(u, mm);
         if (row0 + r < d.nrows)
           for (int c = 0; c < 3; ++c) m[c] = fmax(m[c], mm[c]);
-        for (int c = 0; c < d.nf_out; ++c) res[(c * RB + r) * ld + x] = mk<T>(v[c], T(0));
+        for (int c = 0; c < d.nf_out; ++c) res[c * fs + idx] = mk<T>(v[c], half ? u[c] : T(0));
       }
       if constexpr (Op::kNMax > 0)
         if (op.maxima) block_max_atomic<T, kT>(m[0], m[1], m[2], Op::kNMax, op.maxima);
       __syncthreads();
     }
   }
-  cpx<T>* other = res == A ? B : A;
-  res = gen_fft<T, -1, kT>(res, other, lay, s_tw, nx, d.nf_out * RB, d.nst, d.rad);
+  cpx<T>* other = d.inplace ? res : (res == A ? B : A);
+  res = gen_fft<T, -1, kT>(res, other, lay, s_tw, half ? 2 : 1, M, d.nf_out * RB, -1, d.nst,
+                           d.rad);
   const int n_out = d.nf_out * RB * d.mx_out;
+  const unsigned mx = magic_of(d.mx_out);
   for (int idx = tid; idx < n_out; idx += kT) {
-    const int lr = idx / d.mx_out, k = idx - lr * d.mx_out;
-    const int f = lr / RB, row = row0 + (lr - f * RB);
-    if (row < d.nrows)
-      op.out[f * d.ofs + (long long)row * d.ld_out + k] = scale(res[lr * ld + k], d.scale);
+    const int lr = magic_div(idx, mx, d.mx_out), k = idx - lr * d.mx_out;
+    const int f = magic_div(lr, mRB, RB), row = row0 + (lr - f * RB);
+    if (row >= d.nrows) continue;
+    const cpx<T>* Z = res + lr * M;
+    cpx<T> X = Z[k < M ? k : 0];  // Z[M] = Z[0]
+    if (half) {
+      // X[k] = (Zk + conj Z[M-k]) / 2 + W^k (Zk - conj Z[M-k]) / (2 i)
+      const cpx<T> Zm = conj(Z[k == 0 || k == M ? 0 : M - k]);
+      const cpx<T> w = k == M ? mk<T>(T(-1), T(0)) : s_tw[k];
+      const cpx<T> dd = X - Zm;
+      X = scale((X + Zm) + w * mk<T>(dd.y, -dd.x), T(0.5));
+    }
+    op.out[f * d.ofs + (long long)row * d.ld_out + k] = scale(X, d.scale);
   }
 }
 

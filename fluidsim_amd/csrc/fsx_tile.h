@@ -50,7 +50,7 @@ __device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, unsigned off
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), r, off, 0, 0);
 }
 
-constexpr int kGenThr = 512;  // threads of the mixed-radix tiles
+constexpr int kGenThr = 256;  // threads of the mixed-radix tiles
 
 // Largest tile of a workgroup: 64 KiB (8192 FP32 or 4096 FP64 values); 32
 // KiB for the passes that keep several transforms in registers up to length
@@ -221,14 +221,14 @@ struct StridedDesc {
   int stack;       // outputs of a line stacked as extra lines (OpYInv2NS)
   const cpx<T>* tw;  // exp(-2 pi i m / N), m < N
   // mixed-radix stages of a length without a power-of-two plan (gen_fft)
-  int nst;
+  int nst, inplace;
   int rad[kMaxStages];
 };
 
 // Full transform of one tile of 2^logL lines of length d.N.  LOGN > 0:
 // power-of-two length (tile_fft_p2).  LOGN = 0: any length (gen_fft); slot
 // e of both src and dst is the tile element threadIdx.x + e blockDim.x
-// (line-fast), and the tile uses two LDS buffers.
+// (line-fast), and the tile uses one or two LDS buffers (gen_fft).
 template <typename T, int DIR, int LOGN, int LOGE, class Src, class Dst,
           class Fetch = NoFetch>
 __device__ __forceinline__ void tile_fft(cpx<T>* buf, const cpx<T>* tw,
@@ -240,25 +240,35 @@ __device__ __forceinline__ void tile_fft(cpx<T>* buf, const cpx<T>* tw,
     constexpr int E = 1 << LOGE;
     const int tot = d.N << logL;
     const int lmask = (1 << logL) - 1;
+    const TileLayout lay{1, (1 << logL) | 1};
     cpx<T>* A = buf;
-    cpx<T>* B = buf + tot + (tot >> 5) + 1;
-    const TileLayout lay{logL, 0};
+    cpx<T>* B = d.inplace ? buf : buf + d.N * lay.sp;
+    // all loads of a thread before the first use (slots past the tile repeat
+    // its first element)
+    cpx<T> v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const int idx = threadIdx.x + e * kGenThr;
-      if (idx < tot) A[lpad(idx)] = src(Slot{e, idx & lmask, idx >> logL, 0});
+      const int idx = threadIdx.x + e * kGenThr, q = idx < tot ? idx : 0;
+      v[e] = src(Slot{e, q & lmask, q >> logL, 0});
     }
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int idx = threadIdx.x + e * kGenThr;
-      if (idx < tot) fetch(Slot{e, idx & lmask, idx >> logL, 0});
+      if (idx < tot) A[lay.at(idx & lmask, idx >> logL)] = v[e];
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int idx = threadIdx.x + e * kGenThr, q = idx < tot ? idx : 0;
+      fetch(Slot{e, q & lmask, q >> logL, 0});
     }
     __syncthreads();
-    const cpx<T>* res = gen_fft<T, DIR, kGenThr>(A, B, lay, tw, d.N, 1 << logL, d.nst, d.rad);
+    const cpx<T>* res =
+        gen_fft<T, DIR, kGenThr>(A, B, lay, tw, 1, d.N, 1 << logL, logL, d.nst, d.rad);
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int idx = threadIdx.x + e * kGenThr;
-      if (idx < tot) dst(Slot{e, idx & lmask, idx >> logL, 0}, res[lpad(idx)]);
+      if (idx < tot)
+        dst(Slot{e, idx & lmask, idx >> logL, 0}, res[lay.at(idx & lmask, idx >> logL)]);
     }
     __syncthreads();
   }
@@ -354,8 +364,10 @@ __device__ __forceinline__ cpx<T> ln_load(const Lines& g, const cpx<T>* base, co
     return buf_load<T>(buf_rsrc(base + ln_base<LOGN>(g, s), kBufMax),
                        ln_kept<LOGN>(g, s) ? off : kOOB);
   } else {
-    if (!ln_kept<LOGN>(g, s)) return zero<T>();
-    return base[ln_offset<LOGN>(g, s)];
+    // element 0 is read in place of a masked one: no branch around the load
+    const bool ok = ln_kept<LOGN>(g, s);
+    const cpx<T> v = base[ok ? ln_offset<LOGN>(g, s) : 0];
+    return ok ? v : zero<T>();
   }
 }
 template <int LOGN, typename T>
