@@ -115,6 +115,8 @@ static __global__ __launch_bounds__(64) void k_mfma16_probe(const uint16_t* A, c
   for (int i = 0; i < 16; ++i) D[(8 * (i >> 2) + 4 * g + (i & 3)) * 32 + m] = acc[i];
 }
 
+__device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
+
 // LDS pitches of k_conv_fwd in BF16 elements: odd multiples of 8 (16 bytes),
 // so that the 16-byte reads of 16 consecutive lanes hit distinct banks.
 __host__ __device__ constexpr int odd8(int n) {
@@ -179,8 +181,9 @@ __device__ __forceinline__ void conv_bwd_act_store(const f32x16& acc, const floa
   }
 }
 
-// One workgroup (4 waves) per (image, R output rows); each wave computes
-// 32 output channels x 32 pixels tiles.
+// Form of 8 input channels for more than a few tiles (32 channels:
+// k_conv_strip; few tiles: k_conv_tile). One workgroup (4 waves) per (image,
+// R output rows); each wave computes 32 output channels x 32 pixels tiles.
 // Epilogue: FUSE = 0 writes the FP32 pre-activations y (co_out channels);
 // FUSE = 1 writes the BF16 GELU activations a[p][32] of a hidden layer
 // instead (co_out = 32); FUSE = 2 writes both; FUSE = 3 (input gradient)
@@ -507,6 +510,237 @@ static __global__ __launch_bounds__(512) void k_conv_fwd_run(
   }
 }
 
+// 16-byte accesses of FP32 arrays that need only their own 4-byte alignment
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Epilogue of four output channels co .. co + 3 of one pixel, for the FUSE
+// forms of k_conv_fwd (FUSE != 0: 32 output channels); pre: the layer's
+// pre-activations of FUSE = 3.
+template <int FUSE>
+__device__ __forceinline__ void conv_out4(const float (&acc)[4], const float (&bias)[4], f32x4u pre,
+                                          float* __restrict__ y, uint16_t* __restrict__ a,
+                                          size_t pix, int co) {
+  float v[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = acc[q] + bias[q];
+  if constexpr (FUSE == 0 || FUSE == 2)
+    *reinterpret_cast<f32x4u*>(&y[pix * 32 + co]) = f32x4u{v[0], v[1], v[2], v[3]};
+  if constexpr (FUSE != 0) {
+    uint16_t h[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      h[q] = to_bf16(FUSE == 3 ? v[q] * gelu_grad(pre[q]) : gelu(v[q]));
+    uint2 o;
+    o.x = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
+    o.y = (uint32_t)h[2] | ((uint32_t)h[3] << 16);
+    *reinterpret_cast<uint2*>(&a[pix * 32 + co]) = o;
+  }
+}
+
+// Convolution of 32 input channels without LDS: a wave holds all 50 weight
+// fragments (25 taps x two halves of the channels) in 200 registers and
+// slides down a strip of 32 columns and R output rows. The 10 pixel
+// fragments of an input row (5 column shifts x two halves, 16 bytes per lane
+// from global memory, the shifts hitting L1) serve the five output rows to
+// which the input row contributes, whose accumulators are all live: 50
+// MFMAs per 10 loads, where a form with both operands in LDS reads three
+// operands per two MFMAs and waits at barriers. One wave per SIMD (400 to
+// 480 registers), so the body of an input row is one basic block in which
+// the loads of the next row are in flight during the MFMAs and the epilogue
+// belongs to the output row finished before. To keep that block free of
+// branches the rows past the strip are loaded (wrapped) and multiplied too;
+// their accumulators are dropped. The five accumulators are five independent
+// chains; each takes its taps in the order t, then half.
+// Waves of a workgroup take neighbouring strips of the same rows.
+// 32 images of 128^2: 51 us with FP32 pre-activations and GELU, 47 us as the
+// input gradient (64 and 60 us with both operands in LDS). The MFMAs are
+// 11 us, the bytes 24 us at 4.7 TB/s; the rest is what one wave per SIMD
+// cannot hide: the loads' latency and the epilogue, 16 GELUs per lane and
+// row, which costs as many cycles as the 50 MFMAs (spreading it between them
+// by scheduling groups spilled and was slower, 57 and 54 us).
+template <int FUSE>
+static __global__ __launch_bounds__(256, 1) void k_conv_strip(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+    const float* __restrict__ bias, float* __restrict__ y, int B, int H, int W, int co_out, int R,
+    uint16_t* __restrict__ a_out) {
+  const int lane = threadIdx.x & 63, m = lane & 31, g = lane >> 5;
+  const int nchunk = W / 32, nseg = (H + R - 1) / R;
+  const long long ntask = (long long)B * nseg * nchunk;
+  // consecutive workgroups of an XCD take consecutive tasks (the grid is a
+  // multiple of 8)
+  const int blk = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+  const long long task = (long long)blk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (task >= ntask) return;
+  const int strip = (int)(task % nchunk);
+  const long long rest = task / nchunk;
+  const int seg = (int)(rest % nseg), b = (int)(rest / nseg);
+  const int y0 = seg * R, rows = min(R, H - y0), x0 = strip * 32;
+  u32x4 A[50];
+#pragma unroll
+  for (int s = 0; s < 50; ++s)
+    A[s] = *reinterpret_cast<const u32x4*>(&w[(m * kCnnTaps + s / 2) * 32 + (s % 2) * 16 + 8 * g]);
+  // byte offset in an image row of this lane's pixel under each column shift
+  unsigned off[5];
+#pragma unroll
+  for (int dx = 0; dx < 5; ++dx) {
+    int gx = x0 + m + dx - 2;
+    gx += gx < 0 ? W : (gx >= W ? -W : 0);
+    off[dx] = (unsigned)(gx * 32 + 8 * g) * 2u;
+  }
+  // input row t of the strip is image row y0 - 2 + t, periodic; t is at most
+  // rows + 5 and H at least 4
+  auto load_row = [&](int t, u32x4(&f)[10]) {
+    int gy = y0 - 2 + t;
+    gy += gy < 0 ? H : (gy >= H ? -H : 0);
+    const char* row = reinterpret_cast<const char*>(x + ((size_t)b * H + gy) * W * 32);
+#pragma unroll
+    for (int i = 0; i < 10; ++i)
+      f[i] = *reinterpret_cast<const u32x4*>(row + off[i / 2] + 32 * (i % 2));
+  };
+  float bs[4][4] = {};
+  if constexpr (FUSE != 0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) bs[j][q] = bias[8 * j + 4 * g + q];
+  }
+  const size_t pix0 = ((size_t)b * H + y0) * W + x0 + m;
+  auto fetch = [&](int r, f32x4u(&p)[4]) {
+    if constexpr (FUSE == 3) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        p[j] = *reinterpret_cast<const f32x4u*>(&y[(pix0 + (size_t)r * W) * 32 + 8 * j + 4 * g]);
+    }
+  };
+  f32x16 acc[5];
+  u32x4 cur[10], nxt[10];
+  f32x4u pre[4] = {}, pre_nxt[4] = {};
+  // one input row: output row t - dy is in accumulator (t - dy) mod 5
+  auto mul = [&](int u, int ndy) {
+    acc[u] = f32x16{};
+#pragma unroll
+    for (int i = 0; i < 10; ++i)
+#pragma unroll
+      for (int dy = 0; dy < 5; ++dy)
+        if (dy < ndy) {
+          f32x16& c = acc[(u - dy + 5) % 5];
+          c = mfma16_bf16(as_bf16x8(A[dy * 10 + i]), as_bf16x8(cur[i]), c);
+        }
+#pragma unroll
+    for (int i = 0; i < 10; ++i) cur[i] = nxt[i];
+  };
+  load_row(0, cur);
+#pragma unroll
+  for (int t = 0; t < 5; ++t) {
+    load_row(t + 1, nxt);
+    if (t == 4) fetch(0, pre);
+    mul(t, t + 1);
+  }
+  // input row t = r + 5 with the epilogue of output row r
+  for (int r0 = 0; r0 < rows; r0 += 5) {
+#pragma unroll
+    for (int u = 0; u < 5; ++u) {
+      const int r = r0 + u;
+      if (r >= rows) break;
+      const f32x16 done = acc[u];
+      load_row(r + 6, nxt);
+      fetch(min(r + 1, rows - 1), pre_nxt);
+      mul(u, 5);
+      const size_t pix = pix0 + (size_t)r * W;
+      if constexpr (FUSE == 0) {
+        conv_store_pre(done, bias, y, co_out, pix, g);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float v[4] = {done[4 * j], done[4 * j + 1], done[4 * j + 2], done[4 * j + 3]};
+          conv_out4<FUSE>(v, bs[j], pre[j], y, a_out, pix, 8 * j + 4 * g);
+          pre[j] = pre_nxt[j];
+        }
+      }
+    }
+  }
+}
+
+// Few pixels (one image of 128 x 128 is 512 tiles of 32 pixels): a workgroup
+// of five waves per tile, wave dy multiplying the five taps of kernel row dy
+// (CI = 32: 10 MFMAs; CI = 8: 3, two taps each) straight from global memory,
+// and the partial sums of the waves added in order dy through LDS. The time
+// is a chain of latencies (launch, one round of loads, MFMAs, exchange,
+// epilogue by four waves), not work; the forms that stage weights and pixels
+// in LDS run several such rounds on a third of the waves. One image of
+// 128^2: 6.0 us a hidden layer, 9.6 us with operands staged in LDS.
+template <int CI, int FUSE, bool XF32>
+static __global__ __launch_bounds__(320) void k_conv_tile(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+    const float* __restrict__ bias, float* __restrict__ y, int H, int W, int co_out,
+    uint16_t* __restrict__ a_out) {
+  static_assert(CI == 8 || (CI == 32 && !XF32), "");
+  __shared__ float4 part[5][4][64];
+  const int lane = threadIdx.x & 63, m = lane & 31, g = lane >> 5;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nchunk = W / 32;
+  const int blk = xcd_remap(blockIdx.x, gridDim.x);
+  const int x0 = (blk % nchunk) * 32, row = blk / nchunk;  // row: b H + y
+  const int yy = row % H, b = row / H;
+  int gy = yy + wid - 2;
+  gy += gy < 0 ? H : (gy >= H ? -H : 0);
+  const size_t line = ((size_t)b * H + gy) * W;
+  constexpr int NM = CI == 32 ? 10 : 3;
+  u32x4 A[NM], P[NM];
+#pragma unroll
+  for (int i = 0; i < NM; ++i) {
+    // k of the lane: CI = 32: tap i / 2, channels 16 (i % 2) + 8 g ..;
+    // CI = 8: tap 2 i + g (the sixth is a zero)
+    const int dx = CI == 32 ? i / 2 : 2 * i + g;
+    const int c0 = CI == 32 ? 16 * (i % 2) + 8 * g : 0;
+    A[i] = P[i] = u32x4{0u, 0u, 0u, 0u};
+    if (CI == 32 || dx < 5) {
+      int gx = x0 + m + dx - 2;
+      gx += gx < 0 ? W : (gx >= W ? -W : 0);
+      A[i] = *reinterpret_cast<const u32x4*>(&w[(m * kCnnTaps + wid * 5 + dx) * CI + c0]);
+      if constexpr (XF32)
+        P[i].x = to_bf16(reinterpret_cast<const float*>(x)[line + gx]);
+      else
+        P[i] = *reinterpret_cast<const u32x4*>(&x[(line + gx) * CI + c0]);
+    }
+  }
+  // the epilogue's operands: wave j < 4 takes channels 8 j + 4 g .. + 3
+  const int co = 8 * wid + 4 * g;
+  const size_t pix = (size_t)row * W + x0 + m;
+  float bs[4] = {};
+  f32x4u pre = {};
+  if (wid < 4) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (FUSE != 0 || co + q < co_out) bs[q] = bias[co + q];
+    if constexpr (FUSE == 3) pre = *reinterpret_cast<const f32x4u*>(&y[pix * 32 + co]);
+  }
+  f32x16 acc = {};
+#pragma unroll
+  for (int i = 0; i < NM; ++i) acc = mfma16_bf16(as_bf16x8(A[i]), as_bf16x8(P[i]), acc);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    part[wid][j][lane] = make_float4(acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]);
+  __syncthreads();
+  if (wid >= 4) return;
+  float v[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int dy = 0; dy < 5; ++dy) {
+    const float4 p = part[dy][wid][lane];
+    v[0] += p.x;
+    v[1] += p.y;
+    v[2] += p.z;
+    v[3] += p.w;
+  }
+  if constexpr (FUSE == 0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (co + q < co_out) y[pix * co_out + co + q] = v[q] + bs[q];
+  } else {
+    conv_out4<FUSE>(v, bs, pre, y, a_out, pix, co);
+  }
+}
+
 // wt[c][24 - t][o] = w[o][t][c] for o < co, c < ci; wt has 32 rows and
 // CO_PAD input channels (zero-padded).
 static __global__ void k_conv_flip(const uint16_t* w, int ci, int co, int co_pad, uint16_t* wt) {
@@ -589,8 +823,6 @@ __device__ __forceinline__ void bf16_transpose4x8(const u32x4 (&v)[4], uint2 (&t
     t[2 * d + 1].y = (v[2][d] >> 16) | (v[3][d] & 0xffff0000u);
   }
 }
-
-__device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
 // MFMAs of one 16-pixel chunk: dy operand a, x runs x0 (columns px .. px + 7
 // of the patch) and x1 (px + 8 .. px + 15); tap dx reads px + dx .. + 7.
