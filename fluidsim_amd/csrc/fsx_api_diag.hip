@@ -70,8 +70,11 @@ int diag_geom(const fsx_plan_s* p, int kind, int flags, DiagGeom& g, DiagOut& o,
   if (flags & DIAG_KZKH) off += (long long)Q * g.nkzs * g.nkh;
   o.o_sum = off;
   total = off + Q;
-  // blocks: one kz plane and a run of ky rows each, about 512 blocks
-  int nchunk = (512 + p->nz - 1) / p->nz;
+  // blocks: one kz plane and a run of ky rows each, about 512 blocks (two
+  // per CU, as many as the histograms let live); the means keep sums only,
+  // in about 2048 blocks
+  const int want = kind >= DIAG_NS2D_MEANS ? 2048 : 512;
+  int nchunk = (want + p->nz - 1) / p->nz;
   nchunk = std::max(1, std::min(nchunk, std::max(1, p->ny / 4)));
   g.rows = (p->ny + nchunk - 1) / nchunk;
   g.nchunk = (p->ny + g.rows - 1) / g.rows;

@@ -316,13 +316,15 @@ __device__ __forceinline__ void diag_eval(const DiagIn& in, const Box& b, size_t
 }
 
 // floor bin with linear share; every value at j >= n - 1 goes to n - 1
-__device__ __forceinline__ void share_bin(double k, double dk, int n, int& j, double& c) {
-  j = (int)(k / dk);
+// (inv = 1 / dk; c is continuous across a bin's edge, so a k at an edge may
+// round to either side)
+__device__ __forceinline__ void share_bin(double k, double inv, int n, int& j, double& c) {
+  j = (int)(k * inv);
   if (j >= n - 1) {
     j = n - 1;
     c = 0.0;
   } else {
-    c = (k - j * dk) / dk;
+    c = fma(k, inv, -(double)j);
   }
 }
 
@@ -332,6 +334,11 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// 512^3 FP32 spectra with all five histograms 1344 us, spatial means 435 us
+// (1445 and 535 us with divisions in share_bin, the kx bins of a run on a
+// quarter of the LDS banks, and the means in 512 blocks); the three fields
+// are 1.6 GB, 250 us at the rate of a large read.  The spectra are bound by
+// their FP64 LDS adds, the means by FP64 arithmetic.
 // NT threads per block (waves take the block's ky rows in turn): 256, or
 // 512 for records that leave room for one block per CU
 template <typename T, int KIND, int NT>
@@ -354,6 +361,7 @@ static __global__ __launch_bounds__(NT) void k_diag(DiagIn in, Box box, DiagGeom
   // this lane's copy of the shell / kh histograms: record offset + shift
   const int cp = g.ncopy > 1 ? lane % g.ncopy : 0;
   const int hshift = cp == 0 ? 0 : g.rec + (cp - 1) * span - g.off_k3;
+  const double inv3 = 1.0 / g.dk3, invh = 1.0 / g.dkh;
   Mode m;
   m.ikz = g.dim == 3 ? ksigned(iz, g.nz) : 0;
   m.kz = m.ikz * g.dkz;
@@ -374,6 +382,14 @@ static __global__ __launch_bounds__(NT) void k_diag(DiagIn in, Box box, DiagGeom
   constexpr int kDiagRun = 4;
   constexpr bool kRuns = Q <= 6;
   const bool runs = kRuns && (g.flags & (DIAG_SHELL | DIAG_KZKH)) != 0;
+  // kx histogram: with runs, the lanes' bins of one instruction are kDiagRun
+  // apart, which would put the 64 adds on a quarter of the banks; whole
+  // blocks of 64 kDiagRun bins are kept transposed (r, lane) in LDS
+  const int kx_full = runs ? g.nkxs / (64 * kDiagRun) * (64 * kDiagRun) : 0;
+  auto kx_slot = [&](int ikx) {
+    constexpr int n = 64 * kDiagRun;
+    return ikx < kx_full ? ikx / n * n + ikx % kDiagRun * 64 + ikx % n / kDiagRun : ikx;
+  };
   for (int iy = y0 + wid; iy < y1; iy += nw) {
     m.iky = ksigned(iy, g.ny);
     m.ky = m.iky * g.dky;
@@ -442,18 +458,18 @@ static __global__ __launch_bounds__(NT) void k_diag(DiagIn in, Box box, DiagGeom
 #pragma unroll
         for (int s = 0; s < Q; ++s)
           if (s >= g.q0 && s < g.q0 + g.nq)
-            atomicAdd(&lds[g.off_kx + (s - g.q0) * g.nkxs + ikx], q[s]);
+            atomicAdd(&lds[g.off_kx + (s - g.q0) * g.nkxs + kx_slot(ikx)], q[s]);
       }
       if (g.flags & DIAG_SHELL) {
         int j;
         double c;
-        share_bin(sqrt(mm.k2), g.dk3, g.nk3, j, c);
+        share_bin(sqrt(mm.k2), inv3, g.nk3, j, c);
         accumulate(g.off_k3, g.nk3, j, c, q, js, s0, s1);
       }
       if (g.flags & DIAG_KZKH) {
         int j;
         double c;
-        share_bin(sqrt(mm.kx * mm.kx + mm.ky * mm.ky), g.dkh, g.nkh, j, c);
+        share_bin(sqrt(mm.kx * mm.kx + mm.ky * mm.ky), invh, g.nkh, j, c);
         accumulate(g.off_kh, g.nkh, j, c, q, jh, h0, h1);
       }
     };
@@ -491,7 +507,7 @@ static __global__ __launch_bounds__(NT) void k_diag(DiagIn in, Box box, DiagGeom
         if (g.flags & DIAG_SHELL) {
           int j;
           double c;
-          share_bin(sqrt(m.k2), g.dk3, g.nk3, j, c);
+          share_bin(sqrt(m.k2), inv3, g.nk3, j, c);
 #pragma unroll
           for (int s = 0; s < Q; ++s)
             if (s >= g.q0 && s < g.q0 + g.nq) {
@@ -503,7 +519,7 @@ static __global__ __launch_bounds__(NT) void k_diag(DiagIn in, Box box, DiagGeom
         if (g.flags & DIAG_KZKH) {
           int j;
           double c;
-          share_bin(sqrt(m.kx * m.kx + m.ky * m.ky), g.dkh, g.nkh, j, c);
+          share_bin(sqrt(m.kx * m.kx + m.ky * m.ky), invh, g.nkh, j, c);
 #pragma unroll
           for (int s = 0; s < Q; ++s)
             if (s >= g.q0 && s < g.q0 + g.nq) {
@@ -546,7 +562,11 @@ static __global__ __launch_bounds__(NT) void k_diag(DiagIn in, Box box, DiagGeom
     __syncthreads();
   }
   double* dst = partial + (size_t)blk * g.rec;
-  for (int t = threadIdx.x; t < g.rec; t += blockDim.x) dst[t] = lds[t];
+  for (int t = threadIdx.x; t < g.rec; t += blockDim.x) {
+    const int e = t - g.off_kx;
+    const bool kx = (g.flags & DIAG_KX) && e < g.nq * g.nkxs;
+    dst[t] = lds[kx ? g.off_kx + e / g.nkxs * g.nkxs + kx_slot(e % g.nkxs) : t];
+  }
 }
 
 // Sum of the block records into the output of one quantity group.
