@@ -71,9 +71,13 @@ int diag_geom(const fsx_plan_s* p, int kind, int flags, DiagGeom& g, DiagOut& o,
   o.o_sum = off;
   total = off + Q;
   // blocks: one kz plane and a run of ky rows each, about 512 blocks (two
-  // per CU, as many as the histograms let live); the means keep sums only,
-  // in about 2048 blocks
-  const int want = kind >= DIAG_NS2D_MEANS ? 2048 : 512;
+  // per CU, as many as the histograms let live); the means keep sums only and
+  // take up to 2048 blocks while these have 64 rows or more (below that a
+  // block's start and the longer reduction cost more than they give)
+  const int want =
+      kind >= DIAG_NS2D_MEANS
+          ? (int)std::max(512LL, std::min(2048LL, (long long)p->nz * p->ny / 64))
+          : 512;
   int nchunk = (want + p->nz - 1) / p->nz;
   nchunk = std::max(1, std::min(nchunk, std::max(1, p->ny / 4)));
   g.rows = (p->ny + nchunk - 1) / nchunk;

@@ -562,11 +562,10 @@ static __global__ __launch_bounds__(NT) void k_diag(DiagIn in, Box box, DiagGeom
     __syncthreads();
   }
   double* dst = partial + (size_t)blk * g.rec;
-  for (int t = threadIdx.x; t < g.rec; t += blockDim.x) {
-    const int e = t - g.off_kx;
-    const bool kx = (g.flags & DIAG_KX) && e < g.nq * g.nkxs;
-    dst[t] = lds[kx ? g.off_kx + e / g.nkxs * g.nkxs + kx_slot(e % g.nkxs) : t];
-  }
+  const int nkx_all = kx_full > 0 && (g.flags & DIAG_KX) ? g.nq * g.nkxs : 0;  // off_kx = 0
+  for (int t = threadIdx.x; t < nkx_all; t += blockDim.x)
+    dst[t] = lds[t / g.nkxs * g.nkxs + kx_slot(t % g.nkxs)];
+  for (int t = nkx_all + threadIdx.x; t < g.rec; t += blockDim.x) dst[t] = lds[t];
 }
 
 // Sum of the block records into the output of one quantity group.
