@@ -888,7 +888,7 @@ def bench_closure(args, torch, _lib):
     roofline = {
         "bound": "mfma", "achieved": tflops, "peak": 2500.0, "unit": "TFLOP/s",
         "frac": tflops / 2500.0, "traffic": None,
-        "kernel": f"k_conv_fwd<32, 1>: hidden 32 -> 32 layer on one {nl}^2 field",
+        "kernel": f"k_conv_tile<32, 1>: hidden 32 -> 32 layer on one {nl}^2 field",
         "launch_us": ms.value / max(cnt.value, 1) * 1e3,
         "flops_per_launch": fl.value / max(cnt.value, 1),
         "launches": cnt.value,
