@@ -342,6 +342,10 @@ int launch_strided(Op& op, int N, int nouter, int nlines, int nf, const void* tw
     const size_t lds = ((op.d.inplace ? 1 : 2) * N * ((need / N) | 1) + N) * sizeof(cpx<T>);
     return launch_strided_kernel<T, DIR, 0, LOGE>(op, kGenThr, lds, blocks, nfb, s);
   }
+  // the lanes address 32-bit offsets (fields of 2^31 values and more, beyond
+  // every index of the engine)
+  if (lane_reach(N, LOGE, (unsigned long long)op.pitch(), L, sizeof(cpx<T>)) >= kBufMax)
+    return fail(FSX_ERR_ARG, "field too large for the offsets of a pass");
   switch (logN) {
     case 5: return launch_strided_p2<T, DIR, 5, LOGE>(op, need, blocks, nfb, s);
     case 6: return launch_strided_p2<T, DIR, 6, LOGE>(op, need, blocks, nfb, s);

@@ -20,6 +20,8 @@
 // nx/2) and is where the physical-space products are fused.
 #pragma once
 
+#include <algorithm>
+
 #include "fsx_fft.h"
 #include "fsx_pointwise.h"
 #include "fsx_tile.h"
@@ -69,6 +71,9 @@ void k_strided(Op op) {
   op.template run<DIR, LOGN, LOGE>(buf, s_tw, o, line0);
 }
 
+// An op's pitch() is the larger stride of its two sides (elements between
+// neighbouring positions), for the launcher's check of the lanes' reach.
+//
 // Plain pass: one field per workgroup (blockIdx.y).  The op names the two
 // sides of field f, plane o: geometry (in_lines, out_lines) and base
 // pointers of line line0 (in_base, out_base).
@@ -103,6 +108,7 @@ struct OpZInv : PlainRun<T, OpZInv<T>> {
   long long ifs, ofs;  // field strides (elements)
   int ny, nkx, ld1;
   AxisMap ym, zm;
+  long long pitch() const { return std::max((long long)ny * nkx, (long long)ym.nk() * ld1); }
   static constexpr const unsigned char* mask = nullptr;
   __device__ Lines in_lines(int nl) const {
     return lines_of((unsigned)ny * (unsigned)nkx, zm, false, nl);
@@ -123,6 +129,7 @@ struct OpYInv3 : PlainRun<T, OpYInv3<T>> {
   long long ifs, ofs;
   int ny, ld1, ld2;
   AxisMap ym;
+  long long pitch() const { return ld1 > ld2 ? ld1 : ld2; }
   static constexpr const unsigned char* mask = nullptr;
   __device__ Lines in_lines(int nl) const { return lines_of(ld1, ym, true, nl); }
   __device__ Lines out_lines(int nl) const { return lines_all(ld2, ny, nl); }
@@ -139,6 +146,7 @@ struct OpYFwd3 : PlainRun<T, OpYFwd3<T>> {
   long long ifs, ofs;
   int ny, ld1, ld2;
   AxisMap ym;
+  long long pitch() const { return ld1 > ld2 ? ld1 : ld2; }
   static constexpr const unsigned char* mask = nullptr;
   __device__ Lines in_lines(int nl) const { return lines_all(ld2, ny, nl); }
   __device__ Lines out_lines(int nl) const { return lines_of(ld1, ym, true, nl); }
@@ -157,6 +165,7 @@ struct OpZFwd : PlainRun<T, OpZFwd<T>> {
   int ny, nkx, ld1;
   AxisMap ym, zm;
   const unsigned char* mask;
+  long long pitch() const { return std::max((long long)ny * nkx, (long long)ym.nk() * ld1); }
   __device__ Lines in_lines(int nl) const {
     return lines_all((unsigned)ym.nk() * (unsigned)ld1, zm.n, nl);
   }
@@ -176,6 +185,7 @@ struct OpYInv2 : PlainRun<T, OpYInv2<T>> {
   long long ifs, ofs;
   int nkx, ld2;
   AxisMap ym;
+  long long pitch() const { return nkx > ld2 ? nkx : ld2; }
   static constexpr const unsigned char* mask = nullptr;
   __device__ Lines in_lines(int nl) const { return lines_of(nkx, ym, false, nl); }
   __device__ Lines out_lines(int nl) const { return lines_all(ld2, ym.n, nl); }
@@ -193,6 +203,7 @@ struct OpYFwd2 : PlainRun<T, OpYFwd2<T>> {
   int nkx, ld2;
   AxisMap ym;
   const unsigned char* mask;
+  long long pitch() const { return nkx > ld2 ? nkx : ld2; }
   __device__ Lines in_lines(int nl) const { return lines_all(ld2, ym.n, nl); }
   __device__ Lines out_lines(int nl) const { return lines_of(nkx, ym, false, nl); }
   __device__ long long in_plane(int) const { return 0; }
@@ -220,6 +231,7 @@ struct OpZInvCurl {
   int has_f;
   T fcor;
   int with_b;  // ns3d.strat: input 3 (b) transformed into output 6
+  long long pitch() const { return std::max((long long)ny * nkx, (long long)ym.nk() * ld1); }
 
   template <int DIR, int LOGN, int LOGE>
   __device__ __forceinline__ void run(cpx<T>* buf, const cpx<T>* tw, int o, int line0) const {
@@ -310,6 +322,7 @@ struct OpYInv2NS {
   int ny, nkx, ld2;
   AxisMap ym;
   T dkx, dky;
+  long long pitch() const { return nkx > ld2 ? nkx : ld2; }
 
   // multiplier (without i) of output c at (line, p); applied with
   // scale_rounded, so that the forms of the pass below give the same bits
@@ -345,8 +358,8 @@ struct OpYInv2NS {
             if constexpr (LOGN > 0) {
               // the output field is part of the lane's offset (the launcher
               // stacks only where it fits 32 bits)
-              const unsigned off = ((unsigned)u.j * go.ps + (unsigned)u.line +
-                                    (unsigned)c * (unsigned)ofs) * (unsigned)sizeof(cpx<T>);
+              const unsigned off = ln_lane(go, u, sizeof(cpx<T>)) +
+                                   (unsigned)c * (unsigned)ofs * (unsigned)sizeof(cpx<T>);
               buf_store<T>(buf_rsrc(out0 + ln_base<LOGN>(go, u), kBufMax),
                            ln_kept<LOGN>(go, u) ? off : kOOB, v);
             } else {
@@ -473,6 +486,7 @@ struct OpZFwdRK3 {
   AxisMap ym, zm;
   const unsigned char* mask;
   RKArgs<T> rk;
+  long long pitch() const { return std::max((long long)ny * nkx, (long long)ym.nk() * ld1); }
 
   template <int DIR, int LOGN, int LOGE>
   __device__ __forceinline__ void run(cpx<T>* buf, const cpx<T>* tw, int o, int line0) const {
@@ -531,6 +545,7 @@ struct OpZFwdRKStrat {
   T dkx, dky, dkz;
   T N2;
   RKArgs<T> rk;
+  long long pitch() const { return std::max((long long)ny * nkx, (long long)ym.nk() * ld1); }
 
   template <int DIR, int LOGN, int LOGE>
   __device__ __forceinline__ void run(cpx<T>* buf, const cpx<T>* tw, int o, int line0) const {
@@ -608,6 +623,7 @@ struct OpYFwd2RK {
   // (dt, nu_2, nu_4, nu_8, nu_m4); bpar null: rk.dt and rk.visc
   long long ips = 0, ops = 0;
   const double* bpar = nullptr;
+  long long pitch() const { return nkx > ld2 ? nkx : ld2; }
 
   template <int DIR, int LOGN, int LOGE>
   __device__ __forceinline__ void run(cpx<T>* buf, const cpx<T>* tw, int o, int line0) const {

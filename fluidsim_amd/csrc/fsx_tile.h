@@ -23,8 +23,11 @@ namespace fsx {
 // access whose byte offset is at or beyond the resource's size reads zero
 // and writes nothing, so masked elements (dealiased modes, rows past the
 // end) take the offset kOOB instead of a branch.
-constexpr unsigned kOOB = 0xf8000000u;
-constexpr unsigned kBufMax = 0xf0000000u;  // size given to unbounded resources
+constexpr unsigned kOOB = 0xffe00000u;
+// Size given to resources whose extent is not known (lane_reach: every offset
+// is below it).  4 MiB short of 32 bits: the lanes of a pass over a field of
+// fewer than 2^31 values, the most the element indices reach, stay 8 MiB short.
+constexpr unsigned kBufMax = 0xffc00000u;
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
@@ -65,10 +68,12 @@ constexpr int strided_tile() {
 
 // Register slot of a tile transform: slot number e (stable across calls),
 // local line and position j + pr; pr is a constant of the slot (after
-// unrolling) and a multiple of N / radix, j the rest.
+// unrolling), j the lane's own part: all of the position in mixed-radix
+// tiles, below N / E (E elements per thread) and the same for every slot in
+// power-of-two ones (tile_slot).
 struct Slot {
   int e, line, j, pr;
-  __device__ __forceinline__ int pos() const { return j + pr; }
+  __host__ __device__ __forceinline__ int pos() const { return j + pr; }
 };
 
 // Radix of the stages of a length-2^LOGN transform with 2^LOGE elements per
@@ -98,6 +103,14 @@ struct TilePlan {
   }
   static constexpr int NTW = twoff(NS);
 };
+
+// Slot e of stage S: butterfly j0 + (e / R) N / E, element e % R.
+template <int LOGN, int LOGE, int S>
+__host__ __device__ __forceinline__ Slot tile_slot(int e, int line, int j0) {
+  using PL = TilePlan<LOGN, LOGE>;
+  constexpr int R = 1 << PL::lr(S);
+  return Slot{e, line, j0, (e % R) * (PL::N / R) + (e / R) * (PL::N / PL::E)};
+}
 
 // Copies the stages' twiddles to LDS from tw = exp(-2 pi i m / N).
 template <typename T, int LOGN, int LOGE, int S = 1>
@@ -184,24 +197,22 @@ template <typename T, int DIR, int LOGN, int LOGE, class Src, class Dst, class F
 __device__ __forceinline__ void tile_fft_p2(cpx<T>* buf, const cpx<T>* s_tw, int logL,
                                             Src&& src, Dst&& dst, const Fetch& fetch) {
   using PL = TilePlan<LOGN, LOGE>;
-  constexpr int E = PL::E, N = PL::N;
+  constexpr int E = PL::E;
   const int line = threadIdx.x & ((1 << logL) - 1);
   const int j0 = threadIdx.x >> logL;
   constexpr int R0 = 1 << PL::lr(0);
   cpx<T> v[E];
 #pragma unroll
   for (int e = 0; e < E; ++e)
-    v[e] = src(Slot{e, line, j0 + (e / R0) * (N / E), (e % R0) * (N / R0)});
+    v[e] = src(tile_slot<LOGN, LOGE, 0>(e, line, j0));
 #pragma unroll
   for (int i = 0; i < E / R0; ++i) dftR<T, DIR, R0>(&v[i * R0]);
 #pragma unroll
   for (int e = 0; e < E; ++e)
-    fetch(Slot{e, line, j0 + (e / R0) * (N / E), (e % R0) * (N / R0)});
+    fetch(tile_slot<LOGN, LOGE, 0>(e, line, j0));
   tile_stages<T, DIR, LOGN, LOGE, 1>(v, buf, s_tw, logL, j0, line);
-  constexpr int RL = 1 << PL::lr(PL::NS - 1);
 #pragma unroll
-  for (int e = 0; e < E; ++e)
-    dst(Slot{e, line, j0 + (e / RL) * (N / E), (e % RL) * (N / RL)}, v[e]);
+  for (int e = 0; e < E; ++e) dst(tile_slot<LOGN, LOGE, PL::NS - 1>(e, line, j0), v[e]);
   __syncthreads();
 }
 
@@ -278,11 +289,8 @@ __device__ __forceinline__ void tile_fft(cpx<T>* buf, const cpx<T>* tw,
 template <int LOGN, int LOGE, typename T>
 __device__ __forceinline__ bool last_slot(int e, const StridedDesc<T>& d, int logL, Slot& s) {
   if constexpr (LOGN > 0) {
-    using PL = TilePlan<LOGN, LOGE>;
-    constexpr int RL = 1 << PL::lr(PL::NS - 1);
-    s = Slot{e, (int)threadIdx.x & ((1 << logL) - 1),
-             ((int)threadIdx.x >> logL) + (e / RL) * (PL::N / PL::E),
-             (e % RL) * (PL::N / RL)};
+    s = tile_slot<LOGN, LOGE, TilePlan<LOGN, LOGE>::NS - 1>(
+        e, (int)threadIdx.x & ((1 << logL) - 1), (int)threadIdx.x >> logL);
     return true;
   } else {
     const int idx = threadIdx.x + e * kGenThr;
@@ -303,10 +311,10 @@ struct Lines {
 // all: nothing pruned.  A pruned axis of even length keeps at most n / 2
 // non-negative positions (fsx_plan_create), so every position of the upper
 // half belongs to the upper range.
-__device__ __forceinline__ Lines lines_all(unsigned ps, int n, int nl) {
+__host__ __device__ __forceinline__ Lines lines_all(unsigned ps, int n, int nl) {
   return Lines{ps, n, 0, 0, nl};
 }
-__device__ __forceinline__ Lines lines_of(unsigned ps, const AxisMap& m, bool compact, int nl) {
+__host__ __device__ __forceinline__ Lines lines_of(unsigned ps, const AxisMap& m, bool compact, int nl) {
   if (m.lo + m.hi == m.n) return lines_all(ps, m.n, nl);
   return Lines{ps, m.lo, m.n - m.hi, compact ? m.n - m.lo - m.hi : 0, nl};
 }
@@ -314,8 +322,10 @@ __device__ __forceinline__ Lines lines_of(unsigned ps, const AxisMap& m, bool co
 // An integer the optimizer knows nothing about: comparisons with it stay
 // selects (they would otherwise be threaded into branches around the loads,
 // where a later test repeats them).
-__device__ __forceinline__ int opaque(int x) {
+__host__ __device__ __forceinline__ int opaque(int x) {
+#ifdef __HIP_DEVICE_COMPILE__
   asm("" : "+v"(x));
+#endif
   return x;
 }
 
@@ -331,7 +341,7 @@ __device__ __forceinline__ void pin(cpx<T> (&v)[E]) {
 // Whether slot s is kept on this side.  For power-of-two lengths lines past
 // nl fail both comparisons through an out-of-range j.
 template <int LOGN>
-__device__ __forceinline__ bool ln_kept(const Lines& g, const Slot& s) {
+__host__ __device__ __forceinline__ bool ln_kept(const Lines& g, const Slot& s) {
   if constexpr (LOGN > 0) {
     constexpr int N = 1 << LOGN, H = N / 2;
     return s.pr >= H ? opaque(s.line < g.nl ? s.j : -N) >= g.hi0 - s.pr
@@ -341,11 +351,23 @@ __device__ __forceinline__ bool ln_kept(const Lines& g, const Slot& s) {
     return s.line < g.nl && (p < g.lo || p >= g.hi0);
   }
 }
-// Position offset of the slot's constant part (uniform).
+// Position offset of the slot's constant part (uniform; 64 bits).
 template <int LOGN>
-__device__ __forceinline__ long long ln_base(const Lines& g, const Slot& s) {
+__host__ __device__ __forceinline__ long long ln_base(const Lines& g, const Slot& s) {
   constexpr int H = LOGN > 0 ? 1 << (LOGN - 1) : 1;
   return (long long)(s.pr >= H ? s.pr - g.cut : s.pr) * g.ps;
+}
+// Byte offset of the lane's part, in 32 bits: j and line only, so that it
+// stays below lane_reach.
+__host__ __device__ __forceinline__ unsigned ln_lane(const Lines& g, const Slot& s,
+                                                     unsigned bytes) {
+  return ((unsigned)s.j * g.ps + (unsigned)s.line) * bytes;
+}
+// Largest ln_lane of a power-of-two pass: n / E - 1 positions of pitch ps and
+// the last of nl lines, values of `bytes` bytes.
+inline unsigned long long lane_reach(int n, int loge, unsigned long long ps, int nl,
+                                     unsigned bytes) {
+  return (((unsigned long long)(n >> loge) - 1) * ps + (unsigned)(nl - 1)) * bytes;
 }
 // Element offset of a slot (any length).
 template <int LOGN>
@@ -360,7 +382,7 @@ __device__ __forceinline__ long long ln_offset(const Lines& g, const Slot& s) {
 template <int LOGN, typename T>
 __device__ __forceinline__ cpx<T> ln_load(const Lines& g, const cpx<T>* base, const Slot& s) {
   if constexpr (LOGN > 0) {
-    const unsigned off = ((unsigned)s.j * g.ps + (unsigned)s.line) * (unsigned)sizeof(cpx<T>);
+    const unsigned off = ln_lane(g, s, sizeof(cpx<T>));
     return buf_load<T>(buf_rsrc(base + ln_base<LOGN>(g, s), kBufMax),
                        ln_kept<LOGN>(g, s) ? off : kOOB);
   } else {
@@ -373,7 +395,7 @@ __device__ __forceinline__ cpx<T> ln_load(const Lines& g, const cpx<T>* base, co
 template <int LOGN, typename T>
 __device__ __forceinline__ void ln_store(const Lines& g, cpx<T>* base, const Slot& s, cpx<T> v) {
   if constexpr (LOGN > 0) {
-    const unsigned off = ((unsigned)s.j * g.ps + (unsigned)s.line) * (unsigned)sizeof(cpx<T>);
+    const unsigned off = ln_lane(g, s, sizeof(cpx<T>));
     buf_store<T>(buf_rsrc(base + ln_base<LOGN>(g, s), kBufMax),
                  ln_kept<LOGN>(g, s) ? off : kOOB, v);
   } else {
