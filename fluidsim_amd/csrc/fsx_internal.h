@@ -193,6 +193,21 @@ constexpr int kXThr = 512;       // threads per workgroup of the LDS row pass
 constexpr int kXPassE = 8;       // elements per thread of its tile
 constexpr int kMinBlocks = 1024;  // shrink tiles of small problems below this
 
+// Small problems: power-of-two strided passes of fewer than kSmallWaves waves
+// (4 per CU) with their usual 8 or 16 elements per thread give a thread 4
+// (lengths 2^kSmallLogLo .. 2^kSmallLogHi).  A thread works through its
+// modes one after the other (in the forward passes with a Runge-Kutta
+// stage each has FP64 exponentials), and a pass of one wave per SIMD is as
+// long as that chain.  A Runge-Kutta step of ns2d in a graph with 4 instead of
+// 8 (FP64) or 16 (FP32) elements: 64^2 62 -> 54 us and 83 -> 54, 256^2 79 ->
+// 71 and 96 -> 67, 512^2 100 -> 91 and 112 -> 81, 1024^2 FP32 (860 waves) 175
+// -> 140; ns3d 64^3 175 -> 155 and 145 -> 128, 256 x 256 x 16 262 -> 228 and
+// 203 -> 174 us.  With a limit of 256 waves the last two stay as they were.
+// Fewer lines in a workgroup than fill a wave do not pay on top of that (64^3
+// 155 -> 169 with 8 threads, 160 with 32): their rows are short runs.
+constexpr int kSmallWaves = 1024;
+constexpr int kSmallLogE = 2, kSmallLogLo = 4, kSmallLogHi = 10;
+
 // row stride rounded up to 128 bytes
 template <typename T>
 int padded(int m) {
@@ -254,45 +269,53 @@ int launch_strided_kernel(Op& op, unsigned threads, size_t lds, long long blocks
 // Length-2^LOGN pass: `tile` elements per workgroup, 2^LOGE per thread.
 template <typename T, int DIR, int LOGN, int LOGE, class Op>
 int launch_strided_p2(Op& op, size_t tile, long long blocks, int nfb, hipStream_t s) {
-  const size_t lds =
+  // (a transform of one stage stays in registers)
+  const size_t lds = TilePlan<LOGN, LOGE>::NS == 1 ? 0 :
       (tile + tile / 32 + 1 + TilePlan<LOGN, LOGE>::NTW) * sizeof(cpx<T>);
   return launch_strided_kernel<T, DIR, LOGN, LOGE>(op, (unsigned)(tile >> LOGE), lds, blocks,
                                                    nfb, s);
 }
 
-// Elements per thread of the strided passes: 16 (FP32 passes of one
-// transform per line) or 8 (FP64; passes that keep several transforms of a
-// line in registers).
-template <typename T, class Op>
-constexpr int strided_loge() {
-  return sizeof(T) == 4 && !Op::kMulti ? 4 : 3;
+// The lengths 2^LOGN .. 2^HI with 2^LOGE elements per thread (at most a line).
+template <typename T, int DIR, int LOGE, int LOGN, int HI, class Op>
+int launch_strided_len(Op& op, int logN, size_t tile, long long blocks, int nfb, hipStream_t s) {
+  if constexpr (LOGN <= HI) {
+    if (logN == LOGN)
+      return launch_strided_p2<T, DIR, LOGN, (LOGE < LOGN ? LOGE : LOGN)>(op, tile, blocks, nfb, s);
+    return launch_strided_len<T, DIR, LOGE, LOGN + 1, HI>(op, logN, tile, blocks, nfb, s);
+  } else {
+    return fail(FSX_ERR_ARG, "transform length exceeds the tile");
+  }
 }
+
 template <typename T, int DIR, class Op>
 int launch_strided(Op& op, int N, int nouter, int nlines, int nf, const void* tw,
                    hipStream_t s, bool kio = false, int lines_cap = 0) {
   constexpr int LOGE = strided_loge<T, Op>();
   constexpr int run = 128 / (int)sizeof(cpx<T>);  // lines of a 128-byte run
   const int logN = ilog2(N);
-  const bool p2 = is_pow2(N) && N >= 32;
+  const bool p2 = is_pow2(N);
   const int nfb = Op::kFieldPerBlock ? nf : 1;
-  int L;
+  int loge = std::min(LOGE, logN);
+  size_t most = (size_t)kGenThr << LOGE;  // elements of a workgroup
   if (p2) {
-    const int tile = logN <= 8 ? strided_tile<T, 8, Op>() : strided_tile<T>();
-    if (N > tile) return fail(FSX_ERR_ARG, "transform length exceeds the tile");
-    L = tile / N;
+    if (logN >= kSmallLogLo && logN <= kSmallLogHi &&
+        ((long long)N * nlines * nouter * nfb >> loge) < 64LL * kSmallWaves)
+      loge = std::min(loge, kSmallLogE);
+    most = (size_t)strided_threads<T, Op>(logN, loge) << loge;
     op.d.nst = 0;
   } else {
     // mixed-radix stages in LDS: as many elements as the slots hold
     op.d.nst = gen_factor(N, op.d.rad);
     if (op.d.nst < 0) return fail(FSX_ERR_ARG, "transform length has too many factors");
-    L = (kGenThr << LOGE) / N;
-    if (L < 1) return fail(FSX_ERR_ARG, "transform length exceeds the tile");
   }
+  if ((size_t)N > most) return fail(FSX_ERR_ARG, "transform length exceeds the tile");
+  int L = (int)(most / N);
   while (L & (L - 1)) L &= L - 1;  // power of two
   // fewest lines of a workgroup: a full wave of threads
   int Lmin = 1;
   if (p2)
-    while ((N * Lmin) >> LOGE < 64) Lmin *= 2;
+    while ((N * Lmin) >> loge < 64) Lmin *= 2;
   int cap = 1;
   while (cap < nlines) cap <<= 1;
   if (L > cap) L = cap;
@@ -332,8 +355,7 @@ int launch_strided(Op& op, int N, int nouter, int nlines, int nf, const void* tw
   op.d.stack = 0;
   if constexpr (line_mul<Op>::value > 1) {
     op.d.stack = op.stack_ok() &&
-                 need * line_mul<Op>::value <=
-                     (p2 ? (size_t)strided_tile<T>() : (size_t)kGenThr << LOGE);
+                 need * line_mul<Op>::value <= most;
     if (op.d.stack) need *= line_mul<Op>::value;
   }
 
@@ -344,23 +366,15 @@ int launch_strided(Op& op, int N, int nouter, int nlines, int nf, const void* tw
   }
   // the lanes address 32-bit offsets (fields of 2^31 values and more, beyond
   // every index of the engine)
-  if (lane_reach(N, LOGE, (unsigned long long)op.pitch(), L, sizeof(cpx<T>)) >= kBufMax)
+  if (lane_reach(N, loge, (unsigned long long)op.pitch(), L, sizeof(cpx<T>)) >= kBufMax)
     return fail(FSX_ERR_ARG, "field too large for the offsets of a pass");
-  switch (logN) {
-    case 5: return launch_strided_p2<T, DIR, 5, LOGE>(op, need, blocks, nfb, s);
-    case 6: return launch_strided_p2<T, DIR, 6, LOGE>(op, need, blocks, nfb, s);
-    case 7: return launch_strided_p2<T, DIR, 7, LOGE>(op, need, blocks, nfb, s);
-    case 8: return launch_strided_p2<T, DIR, 8, LOGE>(op, need, blocks, nfb, s);
-    case 9: return launch_strided_p2<T, DIR, 9, LOGE>(op, need, blocks, nfb, s);
-    case 10: return launch_strided_p2<T, DIR, 10, LOGE>(op, need, blocks, nfb, s);
-    case 11: return launch_strided_p2<T, DIR, 11, LOGE>(op, need, blocks, nfb, s);
-    case 12: return launch_strided_p2<T, DIR, 12, LOGE>(op, need, blocks, nfb, s);
-    default:
-      if constexpr (sizeof(T) == 4 && !Op::kMulti) {
-        if (logN == 13) return launch_strided_p2<T, DIR, 13, LOGE>(op, need, blocks, nfb, s);
-      }
-      return fail(FSX_ERR_ARG, "transform length exceeds the tile");
-  }
+  if (loge < std::min(LOGE, logN))
+    return launch_strided_len<T, DIR, kSmallLogE, kSmallLogLo, kSmallLogHi>(op, logN, need, blocks,
+                                                                          nfb, s);
+  // the longest transform fills a tile (1024 threads of 8 elements where
+  // several transforms are kept)
+  constexpr int HI = sizeof(T) == 4 && !Op::kMulti ? 13 : 12;
+  return launch_strided_len<T, DIR, LOGE, 1, HI>(op, logN, need, blocks, nfb, s);
 }
 
 // Row pass of a length nx that is not a power of two (k_xpass_gen).

@@ -44,12 +44,12 @@ __device__ __forceinline__ int xcd_remap(int b, int nb) {
   return x < rem ? x * (q + 1) + local : rem * (q + 1) + (x - rem) * q + local;
 }
 
-// Strided pass.  LOGN > 0: length 2^LOGN, N L / 2^LOGE threads (4 L where
-// the op stacks its outputs); LOGN = 0: any length, kGenThr threads.
+// Strided pass.  LOGN > 0: length 2^LOGN, N L / 2^LOGE threads (4 L lines
+// where the op stacks its outputs); LOGN = 0: any length, kGenThr threads.
 template <typename T, int DIR, int LOGN, int LOGE, class Op>
 // (mixed radix: at least 4, FP64 3, or 2 where transforms are kept, waves per SIMD; the
 // widest of the many butterflies would take 200 to 500 registers otherwise)
-static __global__ __launch_bounds__((LOGN > 0 ? strided_tile<T, LOGN, Op>() >> LOGE : kGenThr),
+static __global__ __launch_bounds__((LOGN > 0 ? strided_threads<T, Op>(LOGN, LOGE) : kGenThr),
                                     (LOGN > 0 ? 1 : (Op::kMulti ? 2 : (sizeof(T) == 8 ? 3 : 4))))
 void k_strided(Op op) {
   extern __shared__ __align__(16) unsigned char smem_raw[];

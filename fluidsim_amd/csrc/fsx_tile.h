@@ -1,18 +1,26 @@
 // Tile transforms of the strided (y and z) passes.
 //
 // A tile is 2^logL adjacent lines (consecutive kx, the contiguous index) of
-// one axis of length N.  Power-of-two lengths from 32 on run tile_fft_p2,
-// whose length is a template argument: the positions a thread touches are
-// then j + constant, so an element costs no index arithmetic beyond one
-// comparison (the kept range of pruned axes) and one LDS address addition.
-// The first version took length and lines as run-time values and spent two
-// thirds of its vector instructions on addresses and branches (512^3 FP32
-// y-inverse: 1243 of them per wave for 450 of arithmetic, issued 67 % of the
-// time; now about 600).  What that gives depends on what else bounds a pass:
-// the y-passes of 512^3 were at the rate of a copy already (y-inverse 814 ->
-// 780 us, 4.6 TB/s), the z-passes with the curl and with the Runge-Kutta
-// stage go from 530 to 508 and from 721 to 671 us, the y-inverse of 256 runs
-// of 128^2 from 35 to 18 us.  Other lengths run gen_fft (mixed radix) in two LDS buffers.
+// one axis of length N.  Power-of-two lengths run tile_fft_p2, whose length is
+// a template argument: the positions a thread touches are then j + constant,
+// so an element costs no index arithmetic beyond one comparison (the kept
+// range of pruned axes) and one LDS address addition.  A version that took
+// length and lines as run-time values spent two thirds of its vector
+// instructions on addresses and branches (512^3 FP32 y-inverse: 1243 of them
+// per wave for 450 of arithmetic, issued 67 % of the time; now about 600).
+// What that gives depends on what else bounds a pass: the y-passes of 512^3
+// were at the rate of a copy already (y-inverse 814 -> 780 us, 4.6 TB/s), the
+// z-passes with the curl and with the Runge-Kutta stage go from 530 to 508 and
+// from 721 to 671 us, the y-inverse of 256 runs of 128^2 from 35 to 18 us.
+//
+// Axes of at most 8 (FP64, several transforms of a line) or 16 points are one
+// stage: each thread transforms a line in registers, without LDS.  A
+// Runge-Kutta step of ns3d on 256 x 256 x 8: 187 us in FP64 and 170 in FP32
+// (629 and 533 with these axes in the mixed-radix stages, 265 and 225 with
+// run-time lengths), on 128 x 128 x 4: 100 and 97 us (749, 647; 174, 154).
+//
+// Other lengths run gen_fft (mixed radix), in one LDS buffer where the
+// butterflies of all threads fit their registers, else in two.
 #pragma once
 
 #include "fsx_fft.h"
@@ -55,15 +63,28 @@ __device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, unsigned off
 
 constexpr int kGenThr = 256;  // threads of the mixed-radix tiles
 
-// Largest tile of a workgroup: 64 KiB (8192 FP32 or 4096 FP64 values); 32
-// KiB for the passes that keep several transforms in registers up to length
-// 256, whose 128-byte runs need no more (512 threads: 256 registers each).
-template <typename T, int LOGN = 0, class Op = void>
+// Largest tile of a workgroup: 64 KiB (8192 FP32 or 4096 FP64 values).
+template <typename T>
 constexpr int strided_tile() {
-  if constexpr (LOGN > 0 && LOGN <= 8 && sizeof(T) == 4) {
-    if (Op::kMulti) return 4096;
-  }
   return sizeof(T) == 4 ? 8192 : 4096;
+}
+// log2 of the elements per thread of the strided passes: 16 (FP32 passes of
+// one transform per line) or 8 (FP64; passes that keep several transforms of
+// a line in registers).
+template <typename T, class Op>
+constexpr int strided_loge() {
+  return sizeof(T) == 4 && !Op::kMulti ? 4 : 3;
+}
+// Threads of a workgroup of a length-2^logn pass with 2^loge elements per
+// thread, at most: a full tile's, half of it for the passes that keep several
+// transforms in registers up to length 256, whose 128-byte runs need no more
+// (512 threads: 256 registers each); where a thread has fewer elements than
+// strided_loge (small problems, short axes), 1024 threads (four stacked lines
+// of 1024), 256 for several transforms.
+template <typename T, class Op>
+constexpr int strided_threads(int logn, int loge) {
+  if (loge < strided_loge<T, Op>()) return Op::kMulti ? 256 : 1024;
+  return (sizeof(T) == 4 && Op::kMulti && logn <= 8 ? 4096 : strided_tile<T>()) >> loge;
 }
 
 // Register slot of a tile transform: slot number e (stable across calls),
@@ -84,7 +105,7 @@ struct TilePlan {
   static constexpr int N = 1 << LOGN;
   static constexpr int E = 1 << LOGE;
   static constexpr int NS = (LOGN + LOGE - 1) / LOGE;
-  static_assert(NS >= 2, "a tile transform has at least two stages");
+  static_assert(NS >= 1 && LOGE <= LOGN, "a thread's elements are of one line");
   static constexpr int lr(int s) {
     const int back = NS - 1 - s;
     const int rank = s <= back ? 2 * s : 2 * back + 1;
@@ -192,7 +213,8 @@ __device__ __forceinline__ void tile_stages(cpx<T> (&v)[1 << LOGE], cpx<T>* buf,
 // fetch(slot) is called for every first-stage slot once its input has been
 // read: a multi-transform pass issues there the global loads of its next
 // transform (same slots), in flight during this one's exchanges.  Ends with
-// a barrier so buf can be reused.
+// a barrier so buf can be reused (a length of at most E is one stage in
+// registers and needs neither).
 template <typename T, int DIR, int LOGN, int LOGE, class Src, class Dst, class Fetch>
 __device__ __forceinline__ void tile_fft_p2(cpx<T>* buf, const cpx<T>* s_tw, int logL,
                                             Src&& src, Dst&& dst, const Fetch& fetch) {
@@ -210,10 +232,10 @@ __device__ __forceinline__ void tile_fft_p2(cpx<T>* buf, const cpx<T>* s_tw, int
 #pragma unroll
   for (int e = 0; e < E; ++e)
     fetch(tile_slot<LOGN, LOGE, 0>(e, line, j0));
-  tile_stages<T, DIR, LOGN, LOGE, 1>(v, buf, s_tw, logL, j0, line);
+  if constexpr (PL::NS > 1) tile_stages<T, DIR, LOGN, LOGE, 1>(v, buf, s_tw, logL, j0, line);
 #pragma unroll
   for (int e = 0; e < E; ++e) dst(tile_slot<LOGN, LOGE, PL::NS - 1>(e, line, j0), v[e]);
-  __syncthreads();
+  if constexpr (PL::NS > 1) __syncthreads();
 }
 
 // Hook of tile_fft after the first stage (default: nothing).
@@ -255,23 +277,35 @@ __device__ __forceinline__ void tile_fft(cpx<T>* buf, const cpx<T>* tw,
     cpx<T>* A = buf;
     cpx<T>* B = d.inplace ? buf : buf + d.N * lay.sp;
     // all loads of a thread before the first use (slots past the tile repeat
-    // its first element)
-    cpx<T> v[E];
+    // its first element).  A tile of up to 256 or 512 elements runs one or two
+    // slots only, as the source may be more than a load: a Runge-Kutta step of
+    // ns2d on 48^2 83 -> 77 us in FP64 and 89 -> 77 in FP32, of ns3d on 48^3
+    // 624 -> 565 and 545 -> 359 us, against all 8 or 16 slots.
+    auto in = [&](auto slots) {
+      constexpr int n = decltype(slots)::value < E ? decltype(slots)::value : E;
+      cpx<T> v[n];
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int idx = threadIdx.x + e * kGenThr, q = idx < tot ? idx : 0;
-      v[e] = src(Slot{e, q & lmask, q >> logL, 0});
-    }
+      for (int e = 0; e < n; ++e) {
+        const int idx = threadIdx.x + e * kGenThr, q = idx < tot ? idx : 0;
+        v[e] = src(Slot{e, q & lmask, q >> logL, 0});
+      }
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int idx = threadIdx.x + e * kGenThr;
-      if (idx < tot) A[lay.at(idx & lmask, idx >> logL)] = v[e];
-    }
+      for (int e = 0; e < n; ++e) {
+        const int idx = threadIdx.x + e * kGenThr;
+        if (idx < tot) A[lay.at(idx & lmask, idx >> logL)] = v[e];
+      }
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int idx = threadIdx.x + e * kGenThr, q = idx < tot ? idx : 0;
-      fetch(Slot{e, q & lmask, q >> logL, 0});
-    }
+      for (int e = 0; e < n; ++e) {
+        const int idx = threadIdx.x + e * kGenThr, q = idx < tot ? idx : 0;
+        fetch(Slot{e, q & lmask, q >> logL, 0});
+      }
+    };
+    if (tot <= kGenThr)
+      in(std::integral_constant<int, 1>());
+    else if (tot <= 2 * kGenThr)
+      in(std::integral_constant<int, 2>());
+    else
+      in(std::integral_constant<int, E>());
     __syncthreads();
     const cpx<T>* res =
         gen_fft<T, DIR, kGenThr>(A, B, lay, tw, 1, d.N, 1 << logL, logL, d.nst, d.rad);
