@@ -49,6 +49,25 @@ METRIC = "RK4 steps/s + %HBM roofline; closure-LES vs DNS speedup at equal error
 PEAK_HBM_GBPS = 8000.0
 KINDS = ["z-pass inverse", "y-pass inverse", "x row pass", "y-pass forward",
          "z-pass forward", "RK stage", "other", "diagnostics pass"]
+# the plane passes (y-inverse, rows, y-forward) of a 3D stage where they overlap
+# on two streams: one block per stage (fsx_timing_read_planes)
+PLANES = "plane passes"
+
+
+def read_timing(_lib, plan):
+    """{name: (ms, bytes, count)} of the launch kinds timed since the last
+    read, which are reset."""
+    ms8 = (_lib.ctypes.c_double * 8)()
+    by8 = (_lib.ctypes.c_double * 8)()
+    cn8 = (_lib.ctypes.c_longlong * 8)()
+    ms, by, cn = _lib.ctypes.c_double(), _lib.ctypes.c_double(), _lib.ctypes.c_longlong()
+    ref = _lib.ctypes.byref
+    _lib.call("fsx_timing_read_planes", plan, ref(ms), ref(by), ref(cn), 0)
+    _lib.call("fsx_timing_read", plan, ms8, by8, cn8, 1)
+    kinds = {KINDS[k]: (ms8[k], by8[k], cn8[k]) for k in range(7) if cn8[k]}
+    if cn.value:
+        kinds[PLANES] = (ms.value, by.value, cn.value)
+    return kinds
 
 
 def b_alg_ns3d(n, prec):
@@ -430,31 +449,27 @@ def bench_strat(args, torch, _lib, copy_gbps):
     torch.cuda.synchronize()
     print(f"[bench] warm-up done, dt = {ts.deltat:.4g}", file=sys.stderr, flush=True)
     _lib.call("fsx_timing_enable", plan, 1)
-    ms8 = (_lib.ctypes.c_double * 8)()
-    by8 = (_lib.ctypes.c_double * 8)()
-    cn8 = (_lib.ctypes.c_longlong * 8)()
-    _lib.call("fsx_timing_read", plan, ms8, by8, cn8, 1)
+    read_timing(_lib, plan)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     for _ in range(args.steps):
         ts.one_time_step()
     torch.cuda.synchronize()
     elapsed = time.perf_counter() - t0
-    _lib.call("fsx_timing_read", plan, ms8, by8, cn8, 1)
+    timed = read_timing(_lib, plan)
     _lib.call("fsx_timing_enable", plan, 0)
     print(f"[bench] timed {args.steps} steps in {elapsed:.3f} s", file=sys.stderr, flush=True)
     steps_per_s = args.steps / elapsed
     kernels = {}
-    for k in range(7):
-        if cn8[k]:
-            kernels[KINDS[k]] = {
-                "avg_ms": ms8[k] / cn8[k],
-                "launches_per_step": cn8[k] / args.steps,
-                "share_of_step": ms8[k] / (elapsed * 1e3),
-                "alg_GBps": by8[k] / (ms8[k] * 1e-3) / 1e9,
-            }
-    dom = max(range(7), key=lambda k: ms8[k])
-    achieved = by8[dom] / (ms8[dom] * 1e-3) / 1e9
+    for name, (ms, by, cn) in timed.items():
+        kernels[name] = {
+            "avg_ms": ms / cn,
+            "launches_per_step": cn / args.steps,
+            "share_of_step": ms / (elapsed * 1e3),
+            "alg_GBps": by / (ms * 1e-3) / 1e9,
+        }
+    dom = max(timed, key=lambda k: timed[k][0])
+    achieved = kernels[dom]["alg_GBps"]
     balg = b_alg_strat(n, prec)
     t_final = ts.t
     del sim, ts
@@ -486,9 +501,9 @@ def bench_strat(args, torch, _lib, copy_gbps):
             "t_after_timed_steps": t_final,
         },
         "roofline": {
-            "bound": "hbm", "kernel": KINDS[dom], "achieved": achieved,
+            "bound": "hbm", "kernel": dom, "achieved": achieved,
             "peak": PEAK_HBM_GBPS, "unit": "GB/s", "frac": achieved / PEAK_HBM_GBPS,
-            "traffic": read_traffic(f"strat_{n}_{args.precision}:{KINDS[dom]}"),
+            "traffic": read_traffic(f"strat_{n}_{args.precision}:{dom}"),
             "copy_peak_measured": copy_gbps, "frac_of_copy": achieved / copy_gbps,
         },
         "step_roofline": {
@@ -1318,10 +1333,7 @@ def main():
     torch.cuda.synchronize()
 
     _lib.call("fsx_timing_enable", plan, 1)
-    ms8 = (_lib.ctypes.c_double * 8)()
-    by8 = (_lib.ctypes.c_double * 8)()
-    cn8 = (_lib.ctypes.c_longlong * 8)()
-    _lib.call("fsx_timing_read", plan, ms8, by8, cn8, 1)
+    read_timing(_lib, plan)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     for _ in range(args.steps):
@@ -1330,26 +1342,25 @@ def main():
         ts.it += 1
     torch.cuda.synchronize()
     elapsed = time.perf_counter() - t0
-    _lib.call("fsx_timing_read", plan, ms8, by8, cn8, 1)
+    timed = read_timing(_lib, plan)
     _lib.call("fsx_timing_enable", plan, 0)
     print(f"[bench] timed {args.steps} steps in {elapsed:.3f} s", file=sys.stderr, flush=True)
 
     steps_per_s = args.steps / elapsed
     diagnostics = time_diagnostics(sim, plan, torch)
     kernels = {}
-    for k in range(7):
-        if cn8[k]:
-            kernels[KINDS[k]] = {
-                "avg_ms": ms8[k] / cn8[k],
-                "launches_per_step": cn8[k] / args.steps,
-                "share_of_step": ms8[k] / (elapsed * 1e3),
-                "alg_GBps": by8[k] / (ms8[k] * 1e-3) / 1e9,
-                "alg_MB_per_launch": by8[k] / cn8[k] / 1e6,
-            }
-    dom = max(range(7), key=lambda k: ms8[k])
-    achieved = by8[dom] / (ms8[dom] * 1e-3) / 1e9
+    for name, (ms, by, cn) in timed.items():
+        kernels[name] = {
+            "avg_ms": ms / cn,
+            "launches_per_step": cn / args.steps,
+            "share_of_step": ms / (elapsed * 1e3),
+            "alg_GBps": by / (ms * 1e-3) / 1e9,
+            "alg_MB_per_launch": by / cn / 1e6,
+        }
+    dom = max(timed, key=lambda k: timed[k][0])
+    achieved = kernels[dom]["alg_GBps"]
     balg = b_alg_ns3d(n, prec)
-    traffic = read_traffic(f"ns3d_{n}_{args.precision}:{KINDS[dom]}")
+    traffic = read_traffic(f"ns3d_{n}_{args.precision}:{dom}")
 
     result = {
         "metric": METRIC,
@@ -1377,13 +1388,13 @@ def main():
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": KINDS[dom],
+            "kernel": dom,
             "achieved": achieved,
             "peak": PEAK_HBM_GBPS,
             "unit": "GB/s",
             "frac": achieved / PEAK_HBM_GBPS,
             "traffic": traffic,
-            "traffic_source": ("HBM bytes per launch of this kernel at this workload from "
+            "traffic_source": ("HBM bytes per launch (block of launches) at this workload from "
                                "rocprofv3 FETCH_SIZE / WRITE_SIZE runs of bench.py, "
                                "committed in profiles/traffic.json (not measured in "
                                "this run)"),

@@ -144,6 +144,10 @@ SIGNATURES = {
         P, ctypes.POINTER(c_double), ctypes.POINTER(c_double),
         ctypes.POINTER(ctypes.c_longlong), c_int,
     ],
+    "fsx_timing_read_planes": [
+        P, ctypes.POINTER(c_double), ctypes.POINTER(c_double),
+        ctypes.POINTER(ctypes.c_longlong), c_int,
+    ],
     "fsx_timing_read": [
         P, ctypes.POINTER(c_double), ctypes.POINTER(c_double),
         ctypes.POINTER(ctypes.c_longlong), c_int,

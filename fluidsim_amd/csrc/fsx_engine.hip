@@ -653,22 +653,31 @@ int fsx_timing_read(fsx_plan p, double* ms, double* bytes, long long* counts,
   return 0;
 }
 
-int fsx_timing_read_network(fsx_plan p, double* ms, double* flops, long long* count,
+static int timing_read_kind(fsx_plan p, int kind, double* ms, double* work, long long* count,
                             int reset) {
-  if (!p || !ms || !flops || !count) return fail(FSX_ERR_ARG, "bad argument");
-  *ms = *flops = 0;
+  if (!p || !ms || !work || !count) return fail(FSX_ERR_ARG, "bad argument");
+  *ms = *work = 0;
   *count = 0;
   if (!p->tm) return 0;
   int rc = tm_flush(p);
   if (rc) return rc;
-  *ms = p->tm->ms[K_CNN];
-  *flops = p->tm->by[K_CNN];
-  *count = p->tm->cnt[K_CNN];
+  *ms = p->tm->ms[kind];
+  *work = p->tm->by[kind];
+  *count = p->tm->cnt[kind];
   if (reset) {
-    p->tm->ms[K_CNN] = p->tm->by[K_CNN] = 0;
-    p->tm->cnt[K_CNN] = 0;
+    p->tm->ms[kind] = p->tm->by[kind] = 0;
+    p->tm->cnt[kind] = 0;
   }
   return 0;
+}
+
+int fsx_timing_read_network(fsx_plan p, double* ms, double* flops, long long* count,
+                            int reset) {
+  return timing_read_kind(p, K_CNN, ms, flops, count, reset);
+}
+
+int fsx_timing_read_planes(fsx_plan p, double* ms, double* bytes, long long* count, int reset) {
+  return timing_read_kind(p, K_PLANES, ms, bytes, count, reset);
 }
 
 }  // extern "C"

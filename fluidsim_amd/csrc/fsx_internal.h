@@ -62,9 +62,11 @@ bool is_pow2(int n) { return n > 0 && (n & (n - 1)) == 0; }
 
 // Live per-kernel timing: HIP events recorded around each pass launch on the
 // stream it runs on, with the algorithmic bytes of that launch (compulsory
-// HBM reads + writes of its inputs and outputs).
+// HBM reads + writes of its inputs and outputs).  Launches that overlap on two
+// streams (ns3d_planes) are timed as one block, from fork to join.
 struct fsx_timing {
-  static constexpr int kKinds = 9;     // kind 8: hidden-layer convolutions
+  // kind 8: hidden-layer convolutions, 9: plane passes in chunks
+  static constexpr int kKinds = 10;
   static constexpr int kReadKinds = 8;  // kinds returned by fsx_timing_read
   bool on = false;
   std::vector<hipEvent_t> ev;  // pairs
@@ -136,12 +138,18 @@ namespace {
 
 // kinds of launches reported by fsx_timing_read
 enum { K_ZINV = 0, K_YINV = 1, K_XPASS = 2, K_YFWD = 3, K_ZFWD = 4, K_RK = 5,
-       K_OTHER = 6, K_DIAG = 7, K_CNN = 8 };
-
+       K_OTHER = 6, K_DIAG = 7, K_CNN = 8, K_PLANES = 9 };
 
 struct PlanScope {
   explicit PlanScope(fsx_plan_s* p) { fsx_g_plan = p; }
   ~PlanScope() { fsx_g_plan = nullptr; }
+};
+
+// No launch is timed by itself while one of these lives (tm_pre, tm_post).
+struct TimedAsOne {
+  fsx_plan_s* p = fsx_g_plan;
+  TimedAsOne() { fsx_g_plan = nullptr; }
+  ~TimedAsOne() { fsx_g_plan = p; }
 };
 
 void note(int kind, double bytes) {
@@ -898,8 +906,11 @@ int ns3d_plane_chunk(fsx_plan_s* p, int z0, int nzc, cpx<T>* w2, int nin, int no
 // between its three passes.  512^3 FP32, three passes of a stage together:
 // 1.99 ms in one go, 1.99 ms in 128 MB chunks on one stream, 1.80 ms in 96 MB
 // chunks on two (2.1 ms in 64 MB chunks: too few workgroups each; 1.99 ms in
-// 128 MB ones: beyond the cache).  Problems whose W2 fits the cache run in
-// one go.
+// 128 MB ones: beyond the cache).  A step: 512^3 12.1 ms in one go, 11.3 in
+// chunks (FP64 24.7, 23.1), ns3d.strat 17.9, 17.1; at 768^3 and 1024^3 a chunk
+// is a few planes and the gain is small (ns3d 116.1, 115.3 and 107.0, 106.7 ms;
+// strat 170.8, 169.5 and 153.9, 152.6).  Problems whose W2 fits the cache run
+// in one go.
 constexpr double kChunkBytes = 96.0 * (1 << 20);
 
 template <typename T>
@@ -913,20 +924,28 @@ int ns3d_planes(fsx_plan_s* p, int nin, int nout, int want_maxima, hipStream_t s
   nchunk += nchunk & 1;
   if (total <= 2 * kChunkBytes || nchunk > p->nz || !p->side)
     return ns3d_plane_chunk<T>(p, 0, p->nz, W2<T>(p), nin, nout, mx, s, strat);
+  int rc = tm_pre(s);
+  if (rc) return rc;
   FSX_HIP(hipEventRecord(p->ev_fork, s));
   FSX_HIP(hipStreamWaitEvent(p->side, p->ev_fork, 0));
-  int rc = 0;
   const int most = (p->nz + nchunk - 1) / nchunk;  // planes of a chunk
-  for (int i = 0; i < nchunk && !rc; ++i) {
-    const int z0 = (int)((long long)p->nz * i / nchunk);
-    const int z1 = (int)((long long)p->nz * (i + 1) / nchunk);
-    rc = ns3d_plane_chunk<T>(p, z0, z1 - z0, W2<T>(p) + (i & 1) * most * plane, nin, nout, mx,
-                             i & 1 ? p->side : s, strat);
+  {
+    TimedAsOne block;
+    for (int i = 0; i < nchunk && !rc; ++i) {
+      const int z0 = (int)((long long)p->nz * i / nchunk);
+      const int z1 = (int)((long long)p->nz * (i + 1) / nchunk);
+      rc = ns3d_plane_chunk<T>(p, z0, z1 - z0, W2<T>(p) + (i & 1) * most * plane, nin, nout, mx,
+                               i & 1 ? p->side : s, strat);
+    }
   }
   // joined on errors too: the side stream's work precedes what follows on s
   FSX_HIP(hipEventRecord(p->ev_join, p->side));
   FSX_HIP(hipStreamWaitEvent(s, p->ev_join, 0));
-  return rc;
+  if (rc) return rc;
+  // y-inverse, rows, y-forward
+  note(K_PLANES, (double)p->nz * g.mx * sizeof(cpx<T>) *
+                     ((nin + nout) * ((double)g.ym.nk() + p->ny) + (nin + nout) * (double)p->ny));
+  return tm_post(s);
 }
 
 // ns3d (strat = 0): z-pass with curl, y-pass, row pass (v x omega, r2c)

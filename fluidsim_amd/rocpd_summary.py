@@ -64,6 +64,23 @@ def dispatch_values(db, counter):
     ).fetchall()
 
 
+def plane_pass_sums(rows):
+    """Counter value of the plane passes (y-inverse, rows, y-forward) of each
+    3D tendency: the sum over the dispatches between the inverse z-pass with
+    the curl and the next z-pass, which are several per pass where the planes
+    run in chunks."""
+    sums, inside = [], False
+    for name, _, val, _ in rows:
+        if "OpZInvCurl" in name:
+            sums.append(0.0)
+            inside = True
+        elif "OpZ" in name:
+            inside = False
+        elif inside and re.search(r"k_xrow|k_xpass|OpYInv3|OpYFwd3", name):
+            sums[-1] += val
+    return sums
+
+
 def traffic(fetch_db, write_db, copy_mib, prefix=""):
     """HBM bytes per dispatch from FETCH_SIZE / WRITE_SIZE (KiB per dispatch),
     each scaled by what the counter reads for the device-to-device copy of
@@ -72,7 +89,8 @@ def traffic(fetch_db, write_db, copy_mib, prefix=""):
     times its 1 GiB device copy before anything else runs; later copies,
     e.g. of whole state fields, have other sizes).  A kernel's value is the
     median over its dispatches (a dispatch whose counters come back short
-    does not drag it down); the range over the dispatches is printed."""
+    does not drag it down); the range over the dispatches is printed.  The
+    plane passes of a 3D tendency are summed as well (plane_pass_sums)."""
     import json
 
     true_kib = copy_mib * 1024.0
@@ -91,6 +109,8 @@ def traffic(fetch_db, write_db, copy_mib, prefix=""):
         agg = defaultdict(list)
         for name, dur, val, grid in rows:
             agg[short_name(name)].append(val)
+        if blocks := plane_pass_sums(rows):
+            agg["plane passes of a tendency"] = blocks
         for name, vals in agg.items():
             v = sorted(vals)
             med = v[len(v) // 2] if len(v) % 2 else 0.5 * (v[len(v) // 2 - 1] + v[len(v) // 2])

@@ -491,6 +491,12 @@ int fsx_timing_read(fsx_plan p, double* ms8, double* bytes8, long long* counts8,
  * reset of fsx_timing_read does too). */
 int fsx_timing_read_network(fsx_plan p, double* ms, double* flops, long long* count,
                             int reset);
+/* fsx_timing_read_planes (sync): the same for the plane passes of a 3D
+ * tendency or stage (y-pass inverse, x row pass, y-pass forward) where they
+ * run in chunks that overlap on two streams: one count per tendency, from the
+ * first chunk's start to the last one's end, and none of these launches in
+ * the kinds 1 to 3 of fsx_timing_read.  reset as above. */
+int fsx_timing_read_planes(fsx_plan p, double* ms, double* bytes, long long* count, int reset);
 
 #ifdef __cplusplus
 }

@@ -77,6 +77,9 @@ CASES = [
     ("fsx_timing_read_network", (None, ctypes.byref(ctypes.c_double()),
                                  ctypes.byref(ctypes.c_double()),
                                  ctypes.byref(ctypes.c_longlong()), 0), "bad argument"),
+    ("fsx_timing_read_planes", (None, ctypes.byref(ctypes.c_double()),
+                                ctypes.byref(ctypes.c_double()),
+                                ctypes.byref(ctypes.c_longlong()), 0), "bad argument"),
     ("fsx_batch_set_lines", (None, 4), "not a batch plan"),
     ("fsx_graph_begin", (None,), "created stream"),
     ("fsx_graph_end", (None, None), "bad argument"),

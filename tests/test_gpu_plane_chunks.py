@@ -94,3 +94,53 @@ def test_chunked_stages_in_a_graph():
         stream.synchronize()
         assert t.equal(eager[0], graph[0]), f"replay {i}"
     _lib.call("fsx_graph_destroy", h)
+
+
+@pytest.mark.parametrize("strat", [False, True])
+def test_timing_of_overlapped_passes(strat):
+    """The plane passes are timed as one block per stage with the bytes of
+    the three passes, the times of all kinds fit into the time of the steps,
+    and a second read after a reset holds nothing."""
+    t = torch()
+    sim = _case(strat)
+    plan = make_plan(sim.oper, 8, 7)
+    S = to_dev_complex(sim.state_spect, 8)
+    tmp, t1 = t.zeros_like(S), t.zeros_like(S)
+    s = _lib.stream_ptr()
+    _lib.call("fsx_set_dt", plan.handle, 1e-3, s)
+    vc = _lib.doubles([1e-3, 0, 0, 0])
+
+    def step():
+        for stage in range(4):
+            bufs = (plan.handle, 4, stage, _lib.dptr(S), _lib.dptr(tmp), _lib.dptr(t1), 0, 0.0)
+            if strat:
+                _lib.call("fsx_strat_rk_stage", *bufs, 4.0, 1, 0, vc, 0.5, 0.2, s)
+            else:
+                _lib.call("fsx_ns3d_rk_stage", *bufs, 1, 0, vc, 0.5, 0.2, s)
+
+    def read():
+        ms, by, cn = ctypes.c_double(), ctypes.c_double(), ctypes.c_longlong()
+        _lib.call("fsx_timing_read_planes", plan.handle, ctypes.byref(ms), ctypes.byref(by),
+                  ctypes.byref(cn), 0)
+        kinds = (ctypes.c_double * 8)(), (ctypes.c_double * 8)(), (ctypes.c_longlong * 8)()
+        _lib.call("fsx_timing_read", plan.handle, *kinds, 1)
+        return ms.value, by.value, cn.value, kinds
+
+    step()
+    _lib.call("fsx_timing_enable", plan.handle, 1)
+    e0, e1 = t.cuda.Event(enable_timing=True), t.cuda.Event(enable_timing=True)
+    e0.record()
+    for _ in range(3):
+        step()
+    e1.record()
+    ms, by, cn, (ms8, by8, cn8) = read()
+    e1.synchronize()
+    assert cn == 12 and list(cn8[1:4]) == [0, 0, 0] and cn8[0] == 12 and cn8[4] == 12
+    kept = sim.oper.where_dealiased == 0
+    mx, nyk = kept.any((0, 1)).sum(), kept.any((0, 2)).sum()
+    nin, nout = (7, 6) if strat else (6, 3)
+    assert by == 12 * 16 * NZ * mx * (nin + nout) * (nyk + 2 * NY)
+    assert 0 < ms and ms + sum(ms8) <= e0.elapsed_time(e1)
+    ms, by, cn, (ms8, by8, cn8) = read()
+    assert ms == by == cn == 0 and sum(ms8) == sum(cn8) == 0
+    _lib.call("fsx_timing_enable", plan.handle, 0)
