@@ -44,31 +44,43 @@ int strip_rows(int B, int H, int W) {
   return best;
 }
 
-// fuse: 0 -> FP32 pre-activations y; 1 -> BF16 GELU activations a (32
-// channels, co_out = 32); 2 -> both; 3 -> a = BF16((conv + bias) GELU'(y))
-// with y the layer's pre-activations (read; co_out = 32)
-template <int CI, int FUSE, bool XF32>
-void conv_fwd_launch(unsigned nblk, size_t lds, hipStream_t s, const uint16_t* x,
-                     const uint16_t* w, const float* bias, float* y, int H, int W, int co_out,
-                     int R, uint16_t* a) {
+// 8 input channels beyond a few tiles (cnn_conv_fwd)
+template <int FUSE, bool XF32>
+int conv_lds_launch(hipStream_t s, const uint16_t* x, const uint16_t* w, const float* bias,
+                    float* y, int B, int H, int W, int co_out, uint16_t* a) {
+  // rows per workgroup: 4 when there are enough workgroups, fewer for
+  // small batches (more workgroups, smaller patches)
+  int R = kCnnRows;
+  while (R > 1 && (long long)B * (H / R) < 512) R >>= 1;
+  const size_t lds = conv_fwd_lds(W, R);
+  if (lds > kLdsMax) return fail(FSX_ERR_ARG, "image too wide for the convolution tile");
+  const unsigned nblk = (unsigned)(B * (H / R));
+  int rc = R >= 2 ? set_lds(k_conv_fwd<FUSE, XF32, 512>, lds)
+                  : set_lds(k_conv_fwd<FUSE, XF32, 256>, lds);
+  if (!rc && R == kCnnRows) rc = set_lds(k_conv_fwd_run<FUSE, XF32>, lds);
+  if (rc) return rc;
+  if ((rc = tm_pre(s))) return rc;
   // 4-row blocks, more than two per CU: the persistent form (weights staged
   // once per workgroup, patch rows in a ring), one workgroup per CU;
   // blocks of 2 rows: 8 waves (more tiles in flight per block; the LDS
   // allows one block per CU), one-row blocks: 4 waves
   const int ncu = cnn_cus();
   if (R == kCnnRows && nblk > 2u * (unsigned)ncu) {
-    const int B = (int)(nblk / (unsigned)(H / R));
     const unsigned grid = (unsigned)(ncu >= 8 ? ncu / 8 * 8 : ncu);
-    hipLaunchKernelGGL((k_conv_fwd_run<CI, FUSE, XF32>), dim3(grid), dim3(512), lds, s, x, w,
-                       bias, y, B, H, W, co_out, a);
+    hipLaunchKernelGGL((k_conv_fwd_run<FUSE, XF32>), dim3(grid), dim3(512), lds, s, x, w, bias, y,
+                       B, H, W, co_out, a);
   } else if (R >= 2)
-    hipLaunchKernelGGL((k_conv_fwd<CI, FUSE, XF32, 512>), dim3(nblk), dim3(512), lds, s, x, w,
-                       bias, y, H, W, co_out, R, a);
+    hipLaunchKernelGGL((k_conv_fwd<FUSE, XF32, 512>), dim3(nblk), dim3(512), lds, s, x, w, bias,
+                       y, H, W, co_out, R, a);
   else
-    hipLaunchKernelGGL((k_conv_fwd<CI, FUSE, XF32, 256>), dim3(nblk), dim3(256), lds, s, x, w,
-                       bias, y, H, W, co_out, R, a);
+    hipLaunchKernelGGL((k_conv_fwd<FUSE, XF32, 256>), dim3(nblk), dim3(256), lds, s, x, w, bias,
+                       y, H, W, co_out, R, a);
+  return 0;
 }
 
+// fuse: 0 -> FP32 pre-activations y; 1 -> BF16 GELU activations a (32
+// channels, co_out = 32); 2 -> both; 3 -> a = BF16((conv + bias) GELU'(y))
+// with y the layer's pre-activations (read; co_out = 32)
 // x_f32: x is one FP32 channel (ci = 8 layer: padded while staged)
 int cnn_conv_fwd(const void* x, int B, int H, int W, int ci, const void* w, const float* bias,
                  int co_out, float* y, hipStream_t s, int fuse = 0, void* a = nullptr,
@@ -82,13 +94,6 @@ int cnn_conv_fwd(const void* x, int B, int H, int W, int ci, const void* w, cons
     return fail(FSX_ERR_ARG, "an FP32 input is one channel (padded to 8) of a hidden layer");
   if (H < kCnnRows || H % kCnnRows || W < 32 || W % 32)
     return fail(FSX_ERR_ARG, "H must be a multiple of 4 and W a multiple of 32");
-  // rows per workgroup: 4 when there are enough workgroups, fewer for
-  // small batches (more workgroups, smaller patches)
-  int R = kCnnRows;
-  while (R > 1 && (long long)B * (H / R) < 512) R >>= 1;
-  const size_t lds = conv_fwd_lds(ci, W, R);
-  if (lds > kLdsMax) return fail(FSX_ERR_ARG, "image too wide for the convolution tile");
-  const unsigned nblk = (unsigned)(B * (H / R));
   const auto* xi = reinterpret_cast<const uint16_t*>(x);
   const auto* wi = reinterpret_cast<const uint16_t*>(w);
   auto* ai = reinterpret_cast<uint16_t*>(a);
@@ -134,21 +139,16 @@ int cnn_conv_fwd(const void* x, int B, int H, int W, int ci, const void* w, cons
     FSX_HIP(hipGetLastError());
     return tm_post(s);
   }
-#define FSX_CONV_FWD(F_, XF_)                                                             \
-  if (fuse == F_ && x_f32 == XF_) {                                                       \
-    rc = R >= 2 ? set_lds(k_conv_fwd<8, F_, XF_, 512>, lds)                               \
-                : set_lds(k_conv_fwd<8, F_, XF_, 256>, lds);                              \
-    if (!rc && R == kCnnRows) rc = set_lds(k_conv_fwd_run<8, F_, XF_>, lds);              \
-    if (rc) return rc;                                                                    \
-    if ((rc = tm_pre(s))) return rc;                                                      \
-    conv_fwd_launch<8, F_, XF_>(nblk, lds, s, xi, wi, bias, y, H, W, co_out, R, ai);      \
-  }
+#define FSX_CONV_FWD(F_, XF_)  \
+  if (fuse == F_ && x_f32 == XF_) \
+    rc = conv_lds_launch<F_, XF_>(s, xi, wi, bias, y, B, H, W, co_out, ai);
   FSX_CONV_FWD(0, false)
   FSX_CONV_FWD(1, false)
   FSX_CONV_FWD(2, false)
   FSX_CONV_FWD(3, false)
   FSX_CONV_FWD(1, true)
 #undef FSX_CONV_FWD
+  if (rc) return rc;
   FSX_HIP(hipGetLastError());
   return tm_post(s);
 }

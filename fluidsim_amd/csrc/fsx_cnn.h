@@ -117,17 +117,16 @@ static __global__ __launch_bounds__(64) void k_mfma16_probe(const uint16_t* A, c
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
-// LDS pitches of k_conv_fwd in BF16 elements: odd multiples of 8 (16 bytes),
-// so that the 16-byte reads of 16 consecutive lanes hit distinct banks.
+// LDS pitches in BF16 elements: odd multiples of 8 (16 bytes), so that the
+// 16-byte reads of 16 consecutive lanes hit distinct banks.
 __host__ __device__ constexpr int odd8(int n) {
   return ((n + 7) / 8) % 2 ? (n + 7) / 8 * 8 : (n + 7) / 8 * 8 + 8;
 }
-__host__ __device__ constexpr int cnn_kp(int ci) { return odd8(kCnnTaps * ci); }
-__host__ __device__ constexpr int cnn_ps(int ci) { return odd8(ci); }
+constexpr int kConvKP = odd8(kCnnTaps * 8);  // weight rows of k_conv_fwd
 
-// LDS bytes of k_conv_fwd: weights [32][KP] + patch [R + 4][W + 4][PS]
-__host__ __device__ inline size_t conv_fwd_lds(int ci, int W, int R) {
-  return (size_t)2 * (32 * cnn_kp(ci) + (size_t)(R + 4) * (W + 4) * cnn_ps(ci));
+// LDS bytes of k_conv_fwd: weights [32][kConvKP] + patch [R + 4][W + 4][8]
+inline size_t conv_fwd_lds(int W, int R) {
+  return (size_t)2 * (32 * kConvKP + (size_t)(R + 4) * (W + 4) * 8);
 }
 
 // Epilogue of FUSE = 3 (input gradient of a hidden layer through the
@@ -189,20 +188,19 @@ __device__ __forceinline__ void conv_bwd_act_store(const f32x16& acc, const floa
 // instead (co_out = 32); FUSE = 2 writes both; FUSE = 3 (input gradient)
 // reads the pre-activations from y and writes BF16 (acc + bias) GELU'(y)
 // to a (co_out = 32).
-// XF32 (CI = 8 only): x is one FP32 channel x[B][H][W], rounded to BF16 and
+// XF32: x is one FP32 channel x[B][H][W], rounded to BF16 and
 // zero-padded to 8 channels while it is staged.
 // NT threads: 256 (4 waves) for one-row blocks, 512 (8 waves, two tiles
 // each per row of 128 columns) for blocks of 2-4 rows
-template <int CI, int FUSE = 0, bool XF32 = false, int NT = 256>
+template <int FUSE = 0, bool XF32 = false, int NT = 256>
 static __global__ __launch_bounds__(NT) void k_conv_fwd(const uint16_t* __restrict__ x,
                                                   const uint16_t* __restrict__ w,
                                                   const float* __restrict__ bias,
                                                   float* __restrict__ y, int H, int W,
                                                   int co_out, int R,
                                                   uint16_t* __restrict__ a_out = nullptr) {
-  constexpr int K = kCnnTaps * CI;
-  constexpr int KP = cnn_kp(CI);
-  constexpr int PS = cnn_ps(CI);
+  constexpr int CI = 8, K = kCnnTaps * CI;
+  constexpr int KP = kConvKP;
   extern __shared__ __align__(16) uint16_t cnn_sm[];
   uint16_t* sw = cnn_sm;
   uint16_t* sp = cnn_sm + 32 * KP;
@@ -210,19 +208,16 @@ static __global__ __launch_bounds__(NT) void k_conv_fwd(const uint16_t* __restri
   const int nyb = H / R;
   const int b = blockIdx.x / nyb, y0 = (blockIdx.x % nyb) * R;
   const int nt = blockDim.x;
-  // Staging: 16-byte global loads and LDS stores (K, CI and both pitches
+  // Staging: 16-byte global loads and LDS stores (K, CI and the weights' pitch
   // are multiples of 8), kLoads weight and kLoads patch loads in flight per
   // thread before the stores. Weights: 32 rows of K. Patch: rows
-  // y0 - 2 .. y0 + R + 1, columns -2 .. W + 1 (periodic), pixels of PS;
-  // element t = (r WP + c) NV + q. A thread's elements are t0 + j nt: q is
-  // fixed (nt is a multiple of NV) and (r, c) advance by nt / NV columns
-  // with a row carry, so no division runs per element.
+  // y0 - 2 .. y0 + R + 1, columns -2 .. W + 1 (periodic), pixels of CI;
+  // element t = r WP + c. A thread's elements are t0 + j nt: (r, c) advance by
+  // nt columns with a row carry, so no division runs per element.
   constexpr int kLoads = 16;
   constexpr int NW16 = 32 * K / 8;
-  constexpr int NV = CI / 8;  // 16-byte vectors per pixel
-  const int NP16 = (R + 4) * WP * NV;
-  const int q = threadIdx.x % NV, cstep = nt / NV;
-  int pc = (threadIdx.x / NV) % WP, pr = (threadIdx.x / NV) / WP;
+  const int NP16 = (R + 4) * WP;
+  int pc = threadIdx.x % WP, pr = threadIdx.x / WP;
   for (int t0 = threadIdx.x; t0 < NW16 || t0 < NP16; t0 += kLoads * nt) {
     u32x4 vw[kLoads], vp[kLoads];
     int off[kLoads];
@@ -230,21 +225,19 @@ static __global__ __launch_bounds__(NT) void k_conv_fwd(const uint16_t* __restri
     for (int j = 0; j < kLoads; ++j) {
       const int t = t0 + j * nt;
       if (t < NW16) vw[j] = reinterpret_cast<const u32x4*>(w)[t];
-      off[j] = (pr * WP + pc) * PS + 8 * q;
+      off[j] = (pr * WP + pc) * CI;
       if (t < NP16) {
         int gy = y0 - 2 + pr, gx = pc - 2;
         gy += gy < 0 ? H : (gy >= H ? -H : 0);
         gx += gx < 0 ? W : (gx >= W ? -W : 0);
         if constexpr (XF32) {
-          static_assert(CI == 8, "one FP32 input channel pads to 8");
           const float v = reinterpret_cast<const float*>(x)[((size_t)b * H + gy) * W + gx];
           vp[j] = u32x4{to_bf16(v), 0u, 0u, 0u};
         } else {
-          vp[j] = *reinterpret_cast<const u32x4*>(
-              &x[(((size_t)b * H + gy) * W + gx) * CI + 8 * q]);
+          vp[j] = *reinterpret_cast<const u32x4*>(&x[(((size_t)b * H + gy) * W + gx) * CI]);
         }
       }
-      pc += cstep;
+      pc += nt;
       while (pc >= WP) {
         pc -= WP;
         ++pr;
@@ -275,7 +268,7 @@ static __global__ __launch_bounds__(NT) void k_conv_fwd(const uint16_t* __restri
       const int tap = k / CI, ci = k % CI;
       const int dy = tap / 5, dx = tap % 5;
       const bf16x8 bb =
-          *reinterpret_cast<const bf16x8*>(&sp[((r + dy) * WP + n0 + m + dx) * PS + ci]);
+          *reinterpret_cast<const bf16x8*>(&sp[((r + dy) * WP + n0 + m + dx) * CI + ci]);
       acc = mfma16_bf16(a, bb, acc);
     }
     if constexpr (K % 16 != 0) {
@@ -286,7 +279,7 @@ static __global__ __launch_bounds__(NT) void k_conv_fwd(const uint16_t* __restri
         const int tap = k / CI, ci = k % CI;
         a = *reinterpret_cast<const bf16x8*>(&sw[m * KP + k]);
         bb = *reinterpret_cast<const bf16x8*>(
-            &sp[((r + tap / 5) * WP + n0 + m + tap % 5) * PS + ci]);
+            &sp[((r + tap / 5) * WP + n0 + m + tap % 5) * CI + ci]);
       }
       acc = mfma16_bf16(a, bb, acc);
     }
@@ -322,7 +315,7 @@ static __global__ __launch_bounds__(NT) void k_conv_fwd(const uint16_t* __restri
 // yu >= -2 in slot (yu + 8) mod 8), so the next row block of the same
 // image stages its 4 new rows only.  Same arithmetic per output as
 // k_conv_fwd.
-template <int CI, int FUSE, bool XF32>
+template <int FUSE, bool XF32>
 static __global__ __launch_bounds__(512) void k_conv_fwd_run(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
     const float* __restrict__ bias, float* __restrict__ y, int B, int H, int W, int co_out,
@@ -330,10 +323,8 @@ static __global__ __launch_bounds__(512) void k_conv_fwd_run(
   constexpr int R = kCnnRows;
   constexpr int NSLOT = R + 4;
   static_assert(NSLOT == 8, "ring of 8 patch rows");
-  constexpr int K = kCnnTaps * CI;
-  constexpr int KP = cnn_kp(CI);
-  constexpr int PS = cnn_ps(CI);
-  constexpr int NV = CI / 8;  // 16-byte vectors per pixel
+  constexpr int CI = 8, K = kCnnTaps * CI;
+  constexpr int KP = kConvKP;
   constexpr int kLoads = 16;
   extern __shared__ __align__(16) uint16_t cnn_sm[];
   uint16_t* sw = cnn_sm;
@@ -386,11 +377,10 @@ static __global__ __launch_bounds__(512) void k_conv_fwd_run(
     have_y0 = y0;
     __syncthreads();  // the previous block's MFMA reads of the ring are done
     {
-      // element t = ((pr - pr0) WP + c) NV + q as in k_conv_fwd, the row
-      // going to its ring slot
-      const int NP16 = (NSLOT - pr0) * WP * NV;
-      const int q = threadIdx.x % NV, cstep = nt / NV;
-      int pc = (threadIdx.x / NV) % WP, pr = pr0 + (threadIdx.x / NV) / WP;
+      // element t = (pr - pr0) WP + c as in k_conv_fwd, the row going to its
+      // ring slot
+      const int NP16 = (NSLOT - pr0) * WP;
+      int pc = threadIdx.x % WP, pr = pr0 + threadIdx.x / WP;
       for (int t0 = threadIdx.x; t0 < NP16; t0 += kLoads * nt) {
         u32x4 vp[kLoads];
         int off[kLoads];
@@ -398,21 +388,19 @@ static __global__ __launch_bounds__(512) void k_conv_fwd_run(
         for (int j = 0; j < kLoads; ++j) {
           const int t = t0 + j * nt;
           const int yu = y0 - 2 + pr;
-          off[j] = (((yu + NSLOT) & (NSLOT - 1)) * WP + pc) * PS + 8 * q;
+          off[j] = (((yu + NSLOT) & (NSLOT - 1)) * WP + pc) * CI;
           if (t < NP16) {
             int gy = yu, gx = pc - 2;
             gy += gy < 0 ? H : (gy >= H ? -H : 0);
             gx += gx < 0 ? W : (gx >= W ? -W : 0);
             if constexpr (XF32) {
-              static_assert(CI == 8, "one FP32 input channel pads to 8");
               const float v = reinterpret_cast<const float*>(x)[((size_t)b * H + gy) * W + gx];
               vp[j] = u32x4{to_bf16(v), 0u, 0u, 0u};
             } else {
-              vp[j] = *reinterpret_cast<const u32x4*>(
-                  &x[(((size_t)b * H + gy) * W + gx) * CI + 8 * q]);
+              vp[j] = *reinterpret_cast<const u32x4*>(&x[(((size_t)b * H + gy) * W + gx) * CI]);
             }
           }
-          pc += cstep;
+          pc += nt;
           while (pc >= WP) {
             pc -= WP;
             ++pr;
@@ -431,7 +419,7 @@ static __global__ __launch_bounds__(512) void k_conv_fwd_run(
     auto bop = [&](int r, int n0, int k) {
       const int tap = k / CI, ci = k % CI;
       const int slot = (ybase + r + tap / 5) & (NSLOT - 1);
-      return *reinterpret_cast<const bf16x8*>(&sp[(slot * WP + n0 + m + tap % 5) * PS + ci]);
+      return *reinterpret_cast<const bf16x8*>(&sp[(slot * WP + n0 + m + tap % 5) * CI + ci]);
     };
     auto epilogue = [&](const f32x16& acc, int r, int n0) {
       const size_t pix = ((size_t)b * H + y0 + r) * W + n0 + m;

@@ -62,3 +62,42 @@ def test_convolution_forms(ci, shape):
               _lib.dptr(d0), s)
     _lib.call("fsx_cnn_conv_bwd_act", *args, _lib.dptr(other), _lib.dptr(d1), s)
     assert torch.equal(d0, d1)
+
+
+@pytest.mark.parametrize("ci, shape", [(32, (1, 4, 288)), (32, (8, 16, 288)), (32, (2, 4, 1216)),
+                                       (8, (2, 4, 1888)), (8, (40, 4, 1152))])
+def test_wide_images(ci, shape):
+    """Widths beyond what the patch rows of an LDS form could hold (at one row
+    per workgroup 276 columns of 32 channels, 1884 of 8) run in the forms
+    without LDS patches, and a wide 8-channel image in the LDS form; same bar as
+    above."""
+    rng = np.random.default_rng(6)
+    B, H, W = shape
+    x = rng.standard_normal(shape + (ci,))
+    w = rng.standard_normal((32, 25, ci)) * 0.2
+    b = rng.standard_normal(32).astype(np.float32)
+    value = lambda a: bf16_value(bf16_bits(a)).astype(np.float64)
+    xd, wd = (torch.from_numpy(bf16_bits(a)).cuda() for a in (x, w))
+    bd = torch.from_numpy(b).cuda()
+    y = torch.full((B, H, W, 32), np.nan, dtype=torch.float32, device="cuda")
+    a = torch.zeros((B, H, W, 32), dtype=torch.int16, device="cuda")
+    args = (_lib.dptr(xd), B, H, W, ci, _lib.dptr(wd), _lib.dptr(bd))
+    _lib.call("fsx_cnn_conv_fwd_act", *args, _lib.dptr(y), _lib.dptr(a), _lib.stream_ptr())
+    pick = sorted({0, B - 1})
+    ref = C.conv(value(x[pick]), value(w), b.astype(np.float64), 32)
+    assert np.abs(y[pick].cpu().numpy() - ref).max() < 1e-5 * np.abs(ref).max()
+    act = torch.zeros_like(a)
+    _lib.call("fsx_cnn_act", _lib.dptr(y), B * H * W, 32, 32, 1, _lib.dptr(act),
+              _lib.stream_ptr())
+    assert torch.equal(act, a)
+
+
+def test_too_wide_for_the_staged_patch():
+    """8 channels beyond a few tiles: the LDS form's width limit."""
+    x = torch.zeros((512, 4, 1216, 8), dtype=torch.int16, device="cuda")
+    w = torch.zeros((32, 25, 8), dtype=torch.int16, device="cuda")
+    b = torch.zeros(32, dtype=torch.float32, device="cuda")
+    y = torch.zeros((512, 4, 1216, 32), dtype=torch.float32, device="cuda")
+    with pytest.raises(ValueError, match="too wide"):
+        _lib.call("fsx_cnn_conv_fwd", _lib.dptr(x), 512, 4, 1216, 8, _lib.dptr(w), _lib.dptr(b),
+                  32, _lib.dptr(y), _lib.stream_ptr())
