@@ -129,11 +129,6 @@ inline size_t conv_fwd_lds(int W, int R) {
   return (size_t)2 * (32 * kConvKP + (size_t)(R + 4) * (W + 4) * 8);
 }
 
-// Epilogue of FUSE = 3 (input gradient of a hidden layer through the
-// activation): a lane's 16 outputs (channels 8 (i / 4) + 4 g + i % 4 of
-// pixel pix) become d = BF16((acc + bias) GELU'(pre)) with the layer's
-// pre-activations pre[pix][32], the value k_cnn_act_bwd computes from the
-// FP32 gradient this replaces.
 // FP32 outputs acc + bias of one lane's pixel: channels 8 j + 4 g .. + 3
 // (j < 4) are contiguous, one 16-byte store each where co_out is a multiple
 // of 4 and y 16-byte aligned, else one store per channel.
@@ -162,6 +157,11 @@ __device__ __forceinline__ void conv_store_pre(const f32x16& acc, const float* b
   }
 }
 
+// Epilogue of FUSE = 3 (input gradient of a hidden layer through the
+// activation): a lane's 16 outputs (channels 8 (i / 4) + 4 g + i % 4 of
+// pixel pix) become d = BF16((acc + bias) GELU'(pre)) with the layer's
+// pre-activations pre[pix][32], the value k_cnn_act_bwd computes from the
+// FP32 gradient this replaces.
 __device__ __forceinline__ void conv_bwd_act_store(const f32x16& acc, const float* bias,
                                                    const float* pre, uint16_t* d, size_t pix,
                                                    int g) {
@@ -181,8 +181,8 @@ __device__ __forceinline__ void conv_bwd_act_store(const f32x16& acc, const floa
 }
 
 // Form of 8 input channels for more than a few tiles (32 channels:
-// k_conv_strip; few tiles: k_conv_tile). One workgroup (4 waves) per (image,
-// R output rows); each wave computes 32 output channels x 32 pixels tiles.
+// k_conv_strip; few tiles: k_conv_tile). One workgroup per (image, R output
+// rows); each wave computes 32 output channels x 32 pixels tiles.
 // Epilogue: FUSE = 0 writes the FP32 pre-activations y (co_out channels);
 // FUSE = 1 writes the BF16 GELU activations a[p][32] of a hidden layer
 // instead (co_out = 32); FUSE = 2 writes both; FUSE = 3 (input gradient)

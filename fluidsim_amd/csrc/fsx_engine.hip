@@ -30,8 +30,9 @@ int fsx_plan_create(fsx_plan* out, int dim, int nx, int ny, int nz, double Lx,
     return fail(FSX_ERR_ARG, "precision must be 4 (float32) or 8 (float64)");
   if (nx < 2 || ny < 2 || (dim == 3 && nz < 2))
     return fail(FSX_ERR_ARG, "grid dimensions must be >= 2");
-  // power-of-two axes: register/LDS Stockham passes; other lengths:
-  // mixed-radix passes with two LDS tile buffers (half the length)
+  // power-of-two axes: register/LDS Stockham passes; other lengths: mixed-radix
+  // passes, whose second LDS buffer (stages that cannot work in place) halves
+  // the longest length
   const int tile = precision == 4 ? strided_tile<float>() : strided_tile<double>();
   auto axis_max = [&](int n) { return is_pow2(n) ? tile : tile / 2; };
   if (ny > axis_max(ny) || nz > axis_max(nz) || (is_pow2(nx) ? nx / 2 > tile : nx > tile / 2))

@@ -4,17 +4,18 @@
 // layout numpy's complex64/complex128 use, so K arrays cross the C-ABI as
 // plain pointers.
 //
-// Transforms are Stockham autosort FFTs of power-of-two length N: radix-R
-// stages (R = 8 while at least three factors of two remain, then 4 or 2).
-// Butterfly j of a stage with sub-transform length Ns reads positions
+// Transforms are Stockham autosort FFTs.  Power-of-two lengths run radix-2 to
+// radix-16 stages: in the strided passes the plan of TilePlan (fsx_tile.h), in
+// the LDS row pass radix 8 while at least three factors of two remain, then 4
+// or 2.  Other lengths: mixed radix, below.  Butterfly j of a stage with sub-transform length Ns reads positions
 // j + r N/R, multiplies input r by W_{Ns R}^{r k} (k = j mod Ns), applies a
 // hard-coded DFT_R and writes output r to (j - k) R + k + r Ns, so the
 // result is in natural order without a bit-reversal pass.
 //
-// The passes keep the first stage in registers (inputs come straight from
-// HBM) and the last stage in registers (outputs go straight to HBM: for the
-// last stage k = j, so output r lands at position j + r Ns); only the middle
-// stages exchange data through LDS.
+// The strided passes of power-of-two lengths keep the first stage in registers
+// (inputs come straight from HBM) and the last stage in registers (outputs go
+// straight to HBM: for the last stage k = j, so output r lands at position
+// j + r Ns); LDS holds only what one stage hands to the next.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -219,7 +219,7 @@ struct OpYFwd2 : PlainRun<T, OpYFwd2<T>> {
 // each input read from HBM once; outputs 0-2 are v, 3-5 omega.
 template <typename T>
 struct OpZInvCurl {
-  static constexpr bool kMulti = true;  // register stashes: half-size tiles
+  static constexpr bool kMulti = true;  // several transforms of a line in registers
   static constexpr bool kFieldPerBlock = false;
   StridedDesc<T> d;
   const cpx<T>* in;  // 3 fields
@@ -655,8 +655,10 @@ struct OpYFwd2RK {
 // ---------------------------------------------------------------- rows
 template <typename T>
 struct XDesc {
-  int nx, lognx, M, logM;  // M = nx / 2 complex points per row
-  int RB, logRB;           // rows per workgroup (power of two)
+  // M complex points per row: nx / 2, odd nx nx; RB rows per workgroup.  The
+  // logarithms are -1 in k_xpass_gen, where M and RB are any numbers
+  int nx, lognx, M, logM;
+  int RB, logRB;
   int nrows;
   int nf_in, nf_out;
   int mx_in, ld_in;    // kept kx and row stride of the c2r input rows
@@ -664,7 +666,7 @@ struct XDesc {
   long long ifs, ofs;  // field strides (elements)
   T scale;             // applied to the r2c output
   const cpx<T>* tw;    // exp(-2 pi i m / nx), m < nx (copied to LDS)
-  // mixed-radix stages of a length-nx complex transform (k_xpass_gen)
+  // mixed-radix stages of a length-M complex transform (k_xpass_gen)
   int nst, inplace;
   int rad[kMaxStages];
 };
