@@ -39,9 +39,6 @@ __device__ __forceinline__ uint16_t to_bf16(float f) {
   const uint32_t u = __float_as_uint(f);
   return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
 }
-__device__ __forceinline__ float from_bf16(uint16_t h) {
-  return __uint_as_float((uint32_t)h << 16);
-}
 
 // GELU, exact (erf) form
 // erf x from e = exp(-x^2): Abramowitz & Stegun, Handbook of Mathematical
