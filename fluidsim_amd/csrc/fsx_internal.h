@@ -256,6 +256,15 @@ struct line_mul<Op, std::void_t<decltype(Op::kLineMul)>> {
   static constexpr int value = Op::kLineMul;
 };
 
+// Ops whose elements per thread follow the waves of one field whatever the
+// fields per launch (OpYInv2NSOne).
+template <class Op, class = void>
+struct per_field { static constexpr bool value = false; };
+template <class Op>
+struct per_field<Op, std::void_t<decltype(Op::kWavesPerField)>> {
+  static constexpr bool value = Op::kWavesPerField;
+};
+
 template <typename T, int DIR, int LOGN, int LOGE, class Op>
 int launch_strided_kernel(Op& op, unsigned threads, size_t lds, long long blocks, int nfb,
                           hipStream_t s) {
@@ -308,7 +317,8 @@ int launch_strided(Op& op, int N, int nouter, int nlines, int nf, const void* tw
   size_t most = (size_t)kGenThr << LOGE;  // elements of a workgroup
   if (p2) {
     if (logN >= kSmallLogLo && logN <= kSmallLogHi &&
-        ((long long)N * nlines * nouter * nfb >> loge) < 64LL * kSmallWaves)
+        ((long long)N * nlines * nouter * (per_field<Op>::value ? 1 : nfb) >> loge) <
+            64LL * kSmallWaves)
       loge = std::min(loge, kSmallLogE);
     most = (size_t)strided_threads<T, Op>(logN, loge) << loge;
     op.d.nst = 0;

@@ -393,6 +393,8 @@ struct OpYInv2NS {
 template <typename T>
 struct OpYInv2NSOne : OpYInv2NS<T> {
   static constexpr bool kFieldPerBlock = true;
+  // the same stages as OpYInv2NS on the same problem: the same bits
+  static constexpr bool kWavesPerField = true;
   static constexpr int kLineMul = 1;
 
   template <int DIR, int LOGN, int LOGE>

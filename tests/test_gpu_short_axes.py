@@ -89,3 +89,24 @@ def test_3d_step(shape, strat, prec):
     args = (0, 0.0, 4.0, 1, 0) if strat else (0, 0.0, 1, 0)
     out = _step(make_plan(oper, prec, 7), S0, prec, name, args)
     assert rel_l2(out, sim.state_spect) < TOL[prec]
+
+
+@pytest.mark.parametrize("prec", [8, 4])
+@pytest.mark.parametrize("n", [512, 1024])
+def test_tile_settings_give_the_same_bits_at_the_small_problem_limit(n, prec):
+    """The elements per thread of a pass do not depend on the tile settings:
+    one output field per workgroup (four times the waves) or all four, any lines
+    per tile, at sizes on both sides of the small-problem limit."""
+    print(f"case tile settings n={n} prec={prec}", flush=True)
+    oper = Oper2D(n, n)
+    plan = make_plan(oper, prec, 4)
+    rot = to_dev_complex(ns2d_noise_rot_fft(n, n, seed=n, kmax=12), prec)
+    outs = []
+    for split, inv, fwd in ((0, 0, 0), (1, 0, 0), (1, 2, 1), (0, 8, 4)):
+        _lib.call("fsx_plan_set_tiles", plan.handle, inv, fwd, split)
+        out = zeros_complex(oper.shapeK, prec)
+        _lib.call("fsx_ns2d_tendency", plan.handle, _lib.dptr(rot), _lib.dptr(out), 0.0, 0,
+                  _lib.stream_ptr())
+        outs.append(host(out))
+    for o in outs[1:]:
+        assert np.array_equal(o, outs[0])
