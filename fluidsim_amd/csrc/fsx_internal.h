@@ -201,21 +201,6 @@ constexpr int kXThr = 512;       // threads per workgroup of the LDS row pass
 constexpr int kXPassE = 8;       // elements per thread of its tile
 constexpr int kMinBlocks = 1024;  // shrink tiles of small problems below this
 
-// Small problems: power-of-two strided passes of fewer than kSmallWaves waves
-// (4 per CU) with their usual 8 or 16 elements per thread give a thread 4
-// (lengths 2^kSmallLogLo .. 2^kSmallLogHi).  A thread works through its
-// modes one after the other (in the forward passes with a Runge-Kutta
-// stage each has FP64 exponentials), and a pass of one wave per SIMD is as
-// long as that chain.  A Runge-Kutta step of ns2d in a graph with 4 instead of
-// 8 (FP64) or 16 (FP32) elements: 64^2 62 -> 54 us and 83 -> 54, 256^2 79 ->
-// 71 and 96 -> 67, 512^2 100 -> 91 and 112 -> 81, 1024^2 FP32 (860 waves) 175
-// -> 140; ns3d 64^3 175 -> 155 and 145 -> 128, 256 x 256 x 16 262 -> 228 and
-// 203 -> 174 us.  With a limit of 256 waves the last two stay as they were.
-// Fewer lines in a workgroup than fill a wave do not pay on top of that (64^3
-// 155 -> 169 with 8 threads, 160 with 32): their rows are short runs.
-constexpr int kSmallWaves = 1024;
-constexpr int kSmallLogE = 2, kSmallLogLo = 4, kSmallLogHi = 10;
-
 // row stride rounded up to 128 bytes
 template <typename T>
 int padded(int m) {
@@ -316,10 +301,8 @@ int launch_strided(Op& op, int N, int nouter, int nlines, int nf, const void* tw
   int loge = std::min(LOGE, logN);
   size_t most = (size_t)kGenThr << LOGE;  // elements of a workgroup
   if (p2) {
-    if (logN >= kSmallLogLo && logN <= kSmallLogHi &&
-        ((long long)N * nlines * nouter * (per_field<Op>::value ? 1 : nfb) >> loge) <
-            64LL * kSmallWaves)
-      loge = std::min(loge, kSmallLogE);
+    loge = small_loge(logN, loge, (long long)nlines * nouter * (per_field<Op>::value ? 1 : nfb),
+                      (unsigned long long)op.pitch(), sizeof(cpx<T>));
     most = (size_t)strided_threads<T, Op>(logN, loge) << loge;
     op.d.nst = 0;
   } else {

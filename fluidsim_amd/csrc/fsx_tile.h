@@ -403,6 +403,30 @@ inline unsigned long long lane_reach(int n, int loge, unsigned long long ps, int
                                      unsigned bytes) {
   return (((unsigned long long)(n >> loge) - 1) * ps + (unsigned)(nl - 1)) * bytes;
 }
+// Small problems: power-of-two strided passes of fewer than kSmallWaves waves
+// (4 per CU) with their usual 8 or 16 elements per thread give a thread 4
+// (lengths 2^kSmallLogLo .. 2^kSmallLogHi).  A thread works through its
+// modes one after the other (in the forward passes with a Runge-Kutta
+// stage each has FP64 exponentials), and a pass of one wave per SIMD is as
+// long as that chain.  A Runge-Kutta step of ns2d in a graph with 4 instead of
+// 8 (FP64) or 16 (FP32) elements: 64^2 62 -> 54 us and 83 -> 54, 256^2 79 ->
+// 71 and 96 -> 67, 512^2 100 -> 91 and 112 -> 81, 1024^2 FP32 (342 waves) 175
+// -> 140; ns3d 64^3 175 -> 155 and 145 -> 128, 256 x 256 x 16 262 -> 228 and
+// 203 -> 174 us.  With a limit of 256 waves the last two stay as they were.
+// Fewer lines in a workgroup than fill a wave do not pay on top of that (64^3
+// 155 -> 169 with 8 threads, 160 with 32): their rows are short runs.
+constexpr int kSmallWaves = 1024;
+constexpr int kSmallLogE = 2, kSmallLogLo = 4, kSmallLogHi = 10;
+// log2 of the elements per thread of a length-2^logn pass over `lines` lines,
+// given the usual one: fewer for a small problem, unless its lanes would reach
+// too far for that (a mask that keeps next to nothing of a large field).
+inline int small_loge(int logn, int loge, long long lines, unsigned long long ps,
+                      unsigned bytes) {
+  if (logn < kSmallLogLo || logn > kSmallLogHi || loge <= kSmallLogE) return loge;
+  if (((lines << logn) >> loge) >= 64LL * kSmallWaves) return loge;
+  // (a tile has at most 1024 lines)
+  return lane_reach(1 << logn, kSmallLogE, ps, 1024, bytes) < kBufMax ? kSmallLogE : loge;
+}
 // Element offset of a slot (any length).
 template <int LOGN>
 __device__ __forceinline__ long long ln_offset(const Lines& g, const Slot& s) {

@@ -32,8 +32,14 @@ template <int LOGN, int LOGE, int S>
 void stage(unsigned bytes) {
   constexpr int N = 1 << LOGN, E = 1 << LOGE;
   const int nl = 16;
-  const unsigned ps = (unsigned)(((1ull << 31) - 1) / N);
-  const int lo = N / 2 - 1, hi = N / 4;  // a pruned axis, in memory or compact
+  // the small form is not taken where its lanes would reach too far
+  unsigned ps = (unsigned)(((1ull << 31) - 1) / N);
+  if (LOGE == kSmallLogE && LOGN > kSmallLogE) {
+    ps /= 4;
+    if (small_loge(LOGN, LOGE + 1, 1, ps, bytes) != LOGE) fail("small form", LOGN, LOGE, bytes);
+  }
+  // a pruned axis, in memory or compact
+  const int lo = N > 2 ? N / 2 - 1 : 1, hi = N / 4;
   const AxisMap whole{N, N / 2 + 1, N / 2 - 1}, pruned{N, lo, hi};
   const Lines sides[3] = {lines_of(ps, whole, false, nl), lines_of(ps, pruned, false, nl),
                           lines_of(ps, pruned, true, nl)};
@@ -73,15 +79,41 @@ void plan(unsigned bytes) {
   stage<LOGN, LOGE, TilePlan<LOGN, LOGE>::NS - 1>(bytes);
 }
 
+// Elements per thread the launcher takes for next to no lines of the largest
+// field, and for many.
+template <int LOGN>
+void chosen(int loge, unsigned bytes) {
+  const unsigned long long ps = ((1ull << 31) - 1) / (1 << LOGN);
+  for (long long lines : {1LL, 1LL << 40}) {
+    const int e = small_loge(LOGN, loge, lines, ps, bytes);
+    if (e > loge || lane_reach(1 << LOGN, e, ps, 16, bytes) >= kBufMax)
+      fail("chosen", LOGN, e, bytes);
+  }
+}
+
 template <int LOGN>
 void length() {
-  plan<LOGN, 3>(8);                     // FP32, several transforms of a line
-  plan<LOGN, 4>(8);                     // FP32
-  if (LOGN <= 12) plan<LOGN, 3>(16);    // FP64
+  constexpr int E3 = LOGN < 3 ? LOGN : 3, E4 = LOGN < 4 ? LOGN : 4;
+  plan<LOGN, E3>(8);                     // FP32, several transforms of a line
+  plan<LOGN, E4>(8);                     // FP32
+  chosen<LOGN>(E3, 8);
+  chosen<LOGN>(E4, 8);
+  if (LOGN <= 12) {
+    plan<LOGN, E3>(16);  // FP64
+    chosen<LOGN>(E3, 16);
+  }
+  if constexpr (LOGN >= kSmallLogLo && LOGN <= kSmallLogHi) {
+    plan<LOGN, kSmallLogE>(8);
+    plan<LOGN, kSmallLogE>(16);
+  }
 }
 
 int main() {
   static_assert(kOOB >= kBufMax && kOOB <= 0xffffffffu - 16, "");
+  length<1>();
+  length<2>();
+  length<3>();
+  length<4>();
   length<5>();
   length<6>();
   length<7>();
