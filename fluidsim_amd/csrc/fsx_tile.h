@@ -277,10 +277,11 @@ __device__ __forceinline__ void tile_fft(cpx<T>* buf, const cpx<T>* tw,
     cpx<T>* A = buf;
     cpx<T>* B = d.inplace ? buf : buf + d.N * lay.sp;
     // all loads of a thread before the first use (slots past the tile repeat
-    // its first element).  A tile of up to 256 or 512 elements runs one or two
-    // slots only, as the source may be more than a load: a Runge-Kutta step of
-    // ns2d on 48^2 83 -> 77 us in FP64 and 89 -> 77 in FP32, of ns3d on 48^3
-    // 624 -> 565 and 545 -> 359 us, against all 8 or 16 slots.
+    // its first element).  A tile of up to 256, 512 or 1024 elements runs one,
+    // two or four slots only, as the source may be more than a load: a
+    // Runge-Kutta step of ns2d on 48^2 83 -> 77 us in FP64 and 89 -> 77 in FP32,
+    // on 100 x 200 103 -> 97 and 108 -> 96, of ns3d on 48^3 624 -> 565 and 545 ->
+    // 359 us, against all 8 or 16 slots.
     auto in = [&](auto slots) {
       constexpr int n = decltype(slots)::value < E ? decltype(slots)::value : E;
       cpx<T> v[n];
@@ -300,10 +301,12 @@ __device__ __forceinline__ void tile_fft(cpx<T>* buf, const cpx<T>* tw,
         fetch(Slot{e, q & lmask, q >> logL, 0});
       }
     };
-    if (tot <= kGenThr)
+    if (tot <= 1 * kGenThr)
       in(std::integral_constant<int, 1>());
     else if (tot <= 2 * kGenThr)
       in(std::integral_constant<int, 2>());
+    else if (tot <= 4 * kGenThr)
+      in(std::integral_constant<int, 4>());
     else
       in(std::integral_constant<int, E>());
     __syncthreads();
